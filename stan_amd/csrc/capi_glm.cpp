@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <chrono>
 #include <cmath>
 #include <cstdlib>
 #include <cstdio>
@@ -679,6 +680,40 @@ int enqueue_pass(sx_glm* m, int propto, int jacobian, bool reduce) {
                            reduce);
 }
 
+// A word of the pinned output that no kernel has stored yet: a NaN with a
+// payload that arithmetic on finite inputs does not produce.
+constexpr uint64_t kUnset = 0x7ff4a5a55a5a0001ull;
+
+void unset_words(double* w, size_t n) {
+  for (size_t i = 0; i < n; ++i) std::memcpy(w + i, &kUnset, sizeof kUnset);
+}
+
+// Waits until the kernels on m's stream have stored n output words (each
+// one aligned 8-byte store, so a word that is no longer kUnset is whole).
+// Watching the words returns a few microseconds before the stream's
+// completion signal would (4 of 20 us for a small evaluation); after 5 ms
+// the stream is waited for instead, which also reports a failed launch.
+int wait_words(sx_glm* m, const double* w, size_t n) {
+  const auto start = std::chrono::steady_clock::now();
+  bool synced = false;
+  unsigned spins = 0;
+  for (size_t i = 0; i < n;) {
+    if (__atomic_load_n(reinterpret_cast<const uint64_t*>(w + i), __ATOMIC_ACQUIRE) != kUnset) {
+      ++i;
+    } else if (synced) {
+      set_error("log_prob: the device stored no result");
+      return SX_EDEVICE;
+    } else if (++spins % 1024 == 0 &&
+               std::chrono::steady_clock::now() - start > std::chrono::milliseconds(5)) {
+      SX_HIP(hipStreamSynchronize(m->stream));
+      synced = true;
+    } else {
+      __builtin_ia32_pause();
+    }
+  }
+  return SX_OK;
+}
+
 int eval(sx_glm* m, const double* theta, int propto, int jacobian, double* lp,
          double* grad) {
   if (!m || !theta || !lp) {
@@ -693,13 +728,25 @@ int eval(sx_glm* m, const double* theta, int propto, int jacobian, double* lp,
       return SX_EDOMAIN;
     }
   std::memcpy(m->h_theta, theta, D * sizeof(double));
-  SX_HIP(hipMemcpyAsync(m->d_theta, m->h_theta, D * sizeof(double), hipMemcpyHostToDevice,
-                        m->stream));
-  int rc = enqueue_pass(m, propto, jacobian);
+  int rc;
+  if (m->family == SX_HIER_LOGIT) {
+    // the last launch (hier_final) starts after the z gradients of the one
+    // before are stored: watch what it stores
+    const size_t head = 2 * static_cast<size_t>(m->K) + 3;
+    unset_words(m->h_out, head);
+    unset_words(m->h_out + D + 1, 1);
+    SX_HIP(hipMemcpyAsync(m->d_theta, m->h_theta, D * sizeof(double), hipMemcpyHostToDevice,
+                          m->stream));
+    rc = sx::hier_enqueue(m, m->hw, m->d_theta, 1, m->h_out, propto, jacobian, false, m->stream,
+                          true);
+    if (rc == SX_OK) rc = wait_words(m, m->h_out, head);
+    if (rc == SX_OK) rc = wait_words(m, m->h_out + D + 1, 1);
+  } else {
+    unset_words(m->h_out, D + 2);
+    rc = sx::plain_eval(m, propto, jacobian);
+    if (rc == SX_OK) rc = wait_words(m, m->h_out, D + 2);
+  }
   if (rc) return rc;
-  SX_HIP(hipMemcpyAsync(m->h_out, m->d_out, (D + 2) * sizeof(double), hipMemcpyDeviceToHost,
-                        m->stream));
-  SX_HIP(hipStreamSynchronize(m->stream));
   *lp = m->h_out[0];
   if (grad) std::memcpy(grad, m->h_out + 1, D * sizeof(double));
   if (m->h_out[D + 1] != 0.0) {
@@ -738,20 +785,15 @@ void free_workspace(hier_workspace& w) {
   w = hier_workspace();
 }
 
-// chains padded to the chain tile of the MFMA kernel (32x32 tiles, waves
-// of 32 chains): 64 for batches of at most 64 chains (two waves per
-// workgroup), else a multiple of 128 (four waves)
-// The FP64 pass of a logistic or normal context: theta (device, D) ->
-// out (device, D + 2), per-block partials in `partials` (blocks x (K + 3)
-// doubles), on `stream`.
-int plain_enqueue(sx_glm* m, const double* d_theta, double* d_out, double* partials, int propto,
-                  int jacobian, hipStream_t stream, bool reduce) {
+// Arguments of the FP64 pass of a logistic or normal context, one chain.
+static pass_args plain_args(const sx_glm* m, const double* theta, double* out, double* partials,
+                            int propto, int jacobian) {
   pass_args a;
   a.X = m->d_X;
   a.y = m->d_y;
-  a.theta = d_theta;
+  a.theta = theta;
   a.partials = partials;
-  a.out = d_out;
+  a.out = out;
   a.N = m->N;
   a.T = m->geom.T;
   a.K = static_cast<int>(m->K);
@@ -770,10 +812,31 @@ int plain_enqueue(sx_glm* m, const double* d_theta, double* d_out, double* parti
   a.alpha_const = a.alpha_sd > 0 ? -std::log(a.alpha_sd) - half_log_2pi : 0.0;
   a.beta_const = a.beta_sd > 0 ? -std::log(a.beta_sd) - half_log_2pi : 0.0;
   a.sigma_const = a.sigma_sd > 0 ? -std::log(a.sigma_sd) - half_log_2pi : 0.0;
+  return a;
+}
+
+// The FP64 pass of a logistic or normal context: theta (device, D) ->
+// out (device, D + 2), per-block partials in `partials` (blocks x (K + 3)
+// doubles), on `stream`.
+int plain_enqueue(sx_glm* m, const double* d_theta, double* d_out, double* partials, int propto,
+                  int jacobian, hipStream_t stream, bool reduce) {
+  const pass_args a = plain_args(m, d_theta, d_out, partials, propto, jacobian);
   SX_HIP(launch_pass_f64(m->family, m->geom, a, m->blocks, m->threads, stream, reduce));
   return SX_OK;
 }
 
+// The same evaluation from h_theta into h_out (pinned, D + 2), whose words
+// the kernels store straight to host memory.
+int plain_eval(sx_glm* m, int propto, int jacobian) {
+  const pass_args a =
+      plain_args(m, m->d_theta, m->h_out, m->d_partials, propto, jacobian);
+  SX_HIP(launch_eval_f64(m->family, m->geom, a, m->h_theta, m->blocks, m->threads, m->stream));
+  return SX_OK;
+}
+
+// chains padded to the chain tile of the MFMA kernel (32x32 tiles, waves
+// of 32 chains): 64 for batches of at most 64 chains (two waves per
+// workgroup), else a multiple of 128 (four waves)
 int mx_chain_pad(const sx_glm* m, int C) {
   (void)m;
   if (C <= 64) return 64;
@@ -969,7 +1032,7 @@ int hier_prepare(sx_glm* m, hier_workspace& w, int C) {
 }
 
 int hier_enqueue(sx_glm* m, hier_workspace& w, const double* d_theta, int C, double* d_out,
-                 int propto, int jacobian, bool fp32, hipStream_t stream) {
+                 int propto, int jacobian, bool fp32, hipStream_t stream, bool host_out) {
   if (fp32 && !m->d_X32 && m->N * m->K > 0) {
     set_error("FP32 evaluation needs a context created with SX_FP32");
     return SX_EINVAL;
@@ -1008,7 +1071,7 @@ int hier_enqueue(sx_glm* m, hier_workspace& w, const double* d_theta, int C, dou
   a.alpha_const = a.alpha_sd > 0 ? -std::log(a.alpha_sd) - h : 0.0;
   a.beta_const = a.beta_sd > 0 ? -std::log(a.beta_sd) - h : 0.0;
   a.tau_const = a.tau_sd > 0 ? -std::log(a.tau_sd) - h : 0.0;
-  SX_HIP(launch_hier(a, fp32, stream));
+  SX_HIP(launch_hier(a, fp32, stream, host_out));
   return SX_OK;
 }
 

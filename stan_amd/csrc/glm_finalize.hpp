@@ -21,14 +21,39 @@ __device__ __forceinline__ double wave_sum(double v) {
   return v;
 }
 
-// Adds priors, Jacobian and scaling to the reduced statistics st[0..E) and
-// writes out[0] = lp, out[1..D] = gradient, out[D+1] = status (0 ok,
-// 1 domain error).  Runs on the first wave of the reduction launch.
-template <int FAM>
-__device__ void finalize(const pass_args& a, const double* st) {
+// Stores one output value.  HOST: `p` is pinned host memory that the host
+// watches while the kernel runs, so the store goes through to it at once
+// (system scope) instead of waiting in this XCD's L2 for the launch's end.
+template <bool HOST>
+__device__ __forceinline__ void put_out(double* p, double v) {
+  if (HOST)
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  else
+    *p = v;
+}
+
+// The gradient of coefficient k: the reduced X^T r entry, scaled, plus the
+// prior (each coefficient on its own, so any thread may do it).
+template <int FAM, bool HOST>
+__device__ __forceinline__ void finalize_beta(const pass_args& a, const double* th, double* out,
+                                              int k, double xtr) {
+  double scale = 1.0;
+  if (FAM == SX_NORMAL) {
+    const double sigma = exp(th[a.K + 1]);
+    scale = 1.0 / (sigma * sigma);
+  }
+  double g = xtr * scale;
+  if (a.beta_sd > 0) g += -th[1 + k] / (a.beta_sd * a.beta_sd);
+  put_out<HOST>(out + 2 + k, g);
+}
+
+// Log density, intercept and scale gradients and the status word from the
+// reduced sum of row terms, sum of residuals and non-finite count; one wave.
+template <int FAM, bool HOST>
+__device__ __forceinline__ void finalize_head(const pass_args& a, const double* th, double* out,
+                                              double sum_term, double sum_r, double bad) {
   const int lane = threadIdx.x & 63;
   const int K = a.K;
-  const double* th = a.theta;
   const double alpha = th[0];
   double lp_prior = 0.0;  // lane-partial of prior terms over beta
   double scale = 1.0;
@@ -36,29 +61,23 @@ __device__ void finalize(const pass_args& a, const double* st) {
     const double sigma = exp(th[K + 1]);
     scale = 1.0 / (sigma * sigma);
   }
-  for (int k = lane; k < K; k += 64) {
-    const double b = th[1 + k];
-    double g = st[2 + k] * scale;
-    if (a.beta_sd > 0) {
-      const double z = b / a.beta_sd;
+  if (a.beta_sd > 0)
+    for (int k = lane; k < K; k += 64) {
+      const double z = th[1 + k] / a.beta_sd;
       lp_prior += -0.5 * z * z;
       if (!a.propto) lp_prior += a.beta_const;
-      g += -b / (a.beta_sd * a.beta_sd);
     }
-    a.out[2 + k] = g;
-  }
   lp_prior = wave_sum(lp_prior);
   if (lane != 0) return;
   double lp = 0.0;
-  double ga = st[1] * scale;
-  double bad = st[K + 2];
+  double ga = sum_r * scale;
   if (FAM == SX_LOGIT) {
-    lp = st[0];
+    lp = sum_term;
   } else {
     const double u = th[K + 1];
     const double sigma = exp(u);
     if (!(sigma > 0) || !isfinite(sigma)) bad += 1.0;
-    const double SS = st[0];
+    const double SS = sum_term;
     lp = -0.5 * SS * scale - static_cast<double>(a.N) * u;
     if (!a.propto) lp += -static_cast<double>(a.N) * kHalfLog2Pi;
     double gu = -static_cast<double>(a.N) + SS * scale;
@@ -73,7 +92,7 @@ __device__ void finalize(const pass_args& a, const double* st) {
       lp += u;
       gu += 1.0;
     }
-    a.out[K + 2] = gu;
+    put_out<HOST>(out + K + 2, gu);
   }
   if (a.alpha_sd > 0) {
     const double z = alpha / a.alpha_sd;
@@ -82,10 +101,19 @@ __device__ void finalize(const pass_args& a, const double* st) {
     ga += -alpha / (a.alpha_sd * a.alpha_sd);
   }
   lp += lp_prior;
-  a.out[0] = lp;
-  a.out[1] = ga;
+  put_out<HOST>(out, lp);
+  put_out<HOST>(out + 1, ga);
   if (!isfinite(lp)) bad += 1.0;
-  a.out[a.D + 1] = bad > 0 ? 1.0 : 0.0;
+  put_out<HOST>(out + a.D + 1, bad > 0 ? 1.0 : 0.0);
+}
+
+// Both, from the reduced statistics in LDS: writes out[0] = lp, out[1..D] =
+// gradient, out[D+1] = status (0 ok, 1 domain error).  Runs on one wave.
+template <int FAM>
+__device__ void finalize(const pass_args& a, const double* st) {
+  for (int k = threadIdx.x & 63; k < a.K; k += 64)
+    finalize_beta<FAM, false>(a, a.theta, a.out, k, st[2 + k]);
+  finalize_head<FAM, false>(a, a.theta, a.out, st[0], st[1], st[a.K + 2]);
 }
 
 }  // namespace

@@ -19,6 +19,7 @@
 
 #include <cmath>
 #include <cstdint>
+#include <type_traits>
 
 #include "../include/stanx/sx_math.hpp"
 #include "glm_finalize.hpp"
@@ -40,6 +41,10 @@ __device__ __forceinline__ double buf_f64(__amdgpu_buffer_rsrc_t r, uint32_t vof
                                           uint32_t soff) {
   return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, voff, soff, 2));
 }
+
+// Blocks of the cross-block reduction per chain: four waves each, wave 0
+// for the log density, the others two columns.
+__host__ __device__ constexpr int reduce_blocks(int K) { return (1 + (K + 1) / 2 + 3) / 4; }
 
 template <int SMAX>
 __device__ __forceinline__ void load_tile(const pass_args& a, int64_t t, int lane,
@@ -67,8 +72,27 @@ __device__ __forceinline__ double load_y(const pass_args& a, int64_t t, int R, i
   }
 }
 
-template <int SMAX, int FAM, int PF>
-__global__ __launch_bounds__(256) void glm_pass_f64(pass_args a) {
+// A single evaluation's theta travels in the kernel arguments (ARG; D <=
+// kThetaArg): the launch itself carries it, where a host-to-device copy
+// would be one more command in the stream with a gap after it.
+struct theta_arg {
+  double v[kThetaArg];
+};
+static_assert(sizeof(pass_args) + sizeof(theta_arg) + 16 <= 4096, "4 KB of kernel arguments");
+struct no_theta {};
+template <bool ARG>
+using theta_of = std::conditional_t<ARG, theta_arg, no_theta>;
+
+template <bool ARG>
+__device__ __forceinline__ const double* theta_ptr(const pass_args& a, const theta_of<ARG>& t) {
+  if constexpr (ARG)
+    return t.v;
+  else
+    return a.theta;
+}
+
+template <int SMAX, int FAM, int PF, bool ARG>
+__global__ __launch_bounds__(256) void glm_pass_f64(pass_args a, theta_of<ARG> ta) {
   extern __shared__ double lds[];
   // 1-D grid of chains x nb blocks.  With nb a multiple of 8 the blocks of
   // every chain that stream the same tiles sit on one XCD (block ids 8
@@ -90,7 +114,8 @@ __global__ __launch_bounds__(256) void glm_pass_f64(pass_args a) {
     blk = __builtin_amdgcn_readfirstlane(blk);
     chain = __builtin_amdgcn_readfirstlane(chain);
   }
-  a.theta += static_cast<int64_t>(chain) * a.theta_stride;
+  const double* theta = theta_ptr<ARG>(a, ta);
+  if constexpr (!ARG) theta += static_cast<int64_t>(chain) * a.theta_stride;
   a.partials += static_cast<int64_t>(chain) * a.E * nb;
   const int lane = threadIdx.x & 63;
   // the wave index is uniform across the wave: say so, so that tile
@@ -103,25 +128,28 @@ __global__ __launch_bounds__(256) void glm_pass_f64(pass_args a) {
   const int R = 64 >> a.lgL;
   const int S = a.S;
 
+  // the first tile's loads are issued before theta is staged: the two
+  // latencies overlap
+  const int64_t W = static_cast<int64_t>(nb) * nw;
+  const int64_t first = static_cast<int64_t>(blk) * nw + wib;
+  int64_t t = first;
+  double xv[SMAX];
+  double yv = 0.0;
+  if (t < a.T) {
+    yv = load_y<FAM>(a, t, R, r);
+    load_tile<SMAX>(a, t, lane, xv);
+  }
   // beta staged in LDS, padded to SMAX*L entries (zero beyond K)
   double* sbeta = lds + nw * a.E;
   for (int i = threadIdx.x; i < SMAX * L; i += blockDim.x)
-    sbeta[i] = i < a.K ? a.theta[1 + i] : 0.0;
+    sbeta[i] = i < a.K ? theta[1 + i] : 0.0;
   __syncthreads();
-  const double alpha = a.theta[0];
+  const double alpha = theta[0];
   double acc[SMAX];
 #pragma unroll
   for (int j = 0; j < SMAX; ++j) acc[j] = 0.0;
   double s0 = 0.0, s1 = 0.0, bad = 0.0;
 
-  const int64_t W = static_cast<int64_t>(nb) * nw;
-  int64_t t = static_cast<int64_t>(blk) * nw + wib;
-  double xv[SMAX];
-  double yv = 0.0;
-  if (PF && t < a.T) {
-    yv = load_y<FAM>(a, t, R, r);
-    load_tile<SMAX>(a, t, lane, xv);
-  }
   for (; t < a.T; t += W) {
     double xn[SMAX];
     double yn = 0.0;
@@ -135,7 +163,7 @@ __global__ __launch_bounds__(256) void glm_pass_f64(pass_args a) {
 #pragma unroll
         for (int j = 0; j < SMAX; ++j) xn[j] = 0.0;
       }
-    } else {
+    } else if (t != first) {
       yv = load_y<FAM>(a, t, R, r);
       load_tile<SMAX>(a, t, lane, xv);
     }
@@ -206,53 +234,68 @@ __global__ __launch_bounds__(256) void glm_pass_f64(pass_args a) {
   }
 }
 
+// Sum over the nb block partials of U entries (rows of nb doubles), in
+// every lane: lane l adds blocks l, l + 64, ... in order, then a fixed
+// shuffle tree.  Eight loads per entry are in flight before the first add;
+// clamped indices and selects keep the loop free of branches.
+template <int U>
+__device__ __forceinline__ void sum_entries(const double* partials, const int (&e)[U], int nb,
+                                            int lane, double (&w)[U]) {
+#pragma unroll
+  for (int u = 0; u < U; ++u) w[u] = 0.0;
+  for (int b0 = 0; b0 < nb; b0 += 512) {
+    double x[U][8];
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int k = 0; k < 8; ++k)
+        x[u][k] = partials[static_cast<int64_t>(e[u]) * nb + min(b0 + lane + 64 * k, nb - 1)];
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int k = 0; k < 8; ++k) w[u] += (b0 + lane + 64 * k < nb) ? x[u][k] : 0.0;
+  }
+#pragma unroll
+  for (int u = 0; u < U; ++u) w[u] = wave_sum(w[u]);
+}
+
 // Cross-block reduction of the bulk pass's partials (fixed order, so the
 // result is bitwise reproducible for a given launch shape) followed by the
 // priors, Jacobian and output.  A separate launch: the kernel boundary
 // makes every block's partials visible without per-block cache
-// write-backs.  One block of 1024 threads; wave w sums entries w, w+16, ...
-template <int FAM>
-__global__ __launch_bounds__(1024) void glm_reduce_f64(pass_args a, int nb) {
-  extern __shared__ double st[];
-  a.theta += static_cast<int64_t>(blockIdx.x) * a.theta_stride;
-  a.partials += static_cast<int64_t>(blockIdx.x) * a.E * nb;
-  a.out += static_cast<int64_t>(blockIdx.x) * a.out_stride;
+// write-backs.  It is bound by latency (211 KB at N = 1e6, K = 100), so the
+// entries are spread over ceil((1 + K / 2) / 4) blocks per chain instead of
+// one (no entry needs another's sum).  Wave 0 takes the log density (row
+// terms, residual sum, non-finite count), every other wave two columns.
+// With theta in the launches and results stored to the host, an evaluation
+// from a host theta takes 24 us at N = 3000, K = 37 (35 with one block and a
+// copy at either end), 40 us at N = 100,003, K = 129 (53) and 135 us at
+// N = 1e6, K = 100 (146, of which the pass 125).
+template <int FAM, bool ARG, bool HOST>
+__global__ __launch_bounds__(256) void glm_reduce_f64(pass_args a, int nb, theta_of<ARG> ta) {
+  const int per = reduce_blocks(a.K);
+  const int chain = static_cast<int>(blockIdx.x) / per;
+  const double* theta = theta_ptr<ARG>(a, ta);
+  if constexpr (!ARG) theta += static_cast<int64_t>(chain) * a.theta_stride;
+  const double* partials = a.partials + static_cast<int64_t>(chain) * a.E * nb;
+  double* out = a.out + static_cast<int64_t>(chain) * a.out_stride;
   const int lane = threadIdx.x & 63;
-  const int wib = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int nw = blockDim.x >> 6;
-  const int E = a.E;
-  // Each wave takes 8 entries per round; every lane issues all of its
-  // loads (8 entries x 4 blocks per step) before any add: clamped indices
-  // and 0/1 weights keep the loop free of branches.
-  for (int i0 = wib * 8; i0 < E; i0 += nw * 8) {
-    double v[8];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) v[u] = 0.0;
-    for (int b0 = 0; b0 < nb; b0 += 256) {
-      double x[8][4];
-#pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        const int i = min(i0 + u, E - 1);
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-          const int b = min(b0 + lane + 64 * k, nb - 1);
-          x[u][k] = a.partials[static_cast<int64_t>(i) * nb + b];
-        }
-      }
-#pragma unroll
-      for (int u = 0; u < 8; ++u)
-#pragma unroll
-        for (int k = 0; k < 4; ++k)
-          v[u] += (b0 + lane + 64 * k < nb) ? x[u][k] : 0.0;
-    }
-#pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      const double w = wave_sum(v[u]);
-      if (lane == 0 && i0 + u < E) st[i0 + u] = w;
-    }
+  const int w = (static_cast<int>(blockIdx.x) - chain * per) * 4 +
+                __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (w == 0) {
+    const int e[3] = {0, 1, a.K + 2};
+    double v[3];
+    sum_entries<3>(partials, e, nb, lane, v);
+    finalize_head<FAM, HOST>(a, theta, out, v[0], v[1], v[2]);
+    return;
   }
-  __syncthreads();
-  if (wib == 0) finalize<FAM>(a, st);
+  const int k = 2 * (w - 1);
+  if (k >= a.K) return;
+  const int e[2] = {2 + k, min(3 + k, a.K + 1)};
+  double v[2];
+  sum_entries<2>(partials, e, nb, lane, v);
+  if (lane < 2 && k + lane < a.K)
+    finalize_beta<FAM, HOST>(a, theta, out, k + lane, lane == 0 ? v[0] : v[1]);
 }
 
 __global__ void tile_x_f64(const double* __restrict__ Xrm, double* __restrict__ Xt,
@@ -268,34 +311,62 @@ __global__ void tile_x_f64(const double* __restrict__ Xrm, double* __restrict__ 
   Xt[idx] = (row < N && col < K) ? Xrm[row * K + col] : 0.0;
 }
 
-template <int SMAX, int FAM, int PF>
-hipError_t launch_one(const pass_args& a, int blocks, int threads, hipStream_t s,
-                      bool reduce) {
+template <int SMAX, int FAM, int PF, bool ARG>
+void launch_one(const pass_args& a, const theta_of<ARG>& ta, int blocks, int threads,
+                hipStream_t s) {
   const size_t lds =
       (static_cast<size_t>(threads / 64) * a.E + static_cast<size_t>(SMAX) * a.L) * sizeof(double);
-  hipLaunchKernelGGL((glm_pass_f64<SMAX, FAM, PF>), dim3(blocks * a.chains), dim3(threads),
-                     lds, s, a);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess || !reduce) return e;
-  hipLaunchKernelGGL((glm_reduce_f64<FAM>), dim3(a.chains), dim3(1024), a.E * sizeof(double),
-                     s, a, blocks);
+  hipLaunchKernelGGL((glm_pass_f64<SMAX, FAM, PF, ARG>), dim3(blocks * a.chains), dim3(threads),
+                     lds, s, a, ta);
+}
+
+template <int FAM, int PF, bool ARG>
+hipError_t launch_fam(int smax, const pass_args& a, const theta_of<ARG>& ta, int blocks,
+                      int threads, hipStream_t s) {
+  switch (smax) {
+    case 4: launch_one<4, FAM, PF, ARG>(a, ta, blocks, threads, s); break;
+    case 8: launch_one<8, FAM, PF, ARG>(a, ta, blocks, threads, s); break;
+    case 12: launch_one<12, FAM, PF, ARG>(a, ta, blocks, threads, s); break;
+    case 16: launch_one<16, FAM, PF, ARG>(a, ta, blocks, threads, s); break;
+    case 20: launch_one<20, FAM, PF, ARG>(a, ta, blocks, threads, s); break;
+    case 24: launch_one<24, FAM, PF, ARG>(a, ta, blocks, threads, s); break;
+    case 28: launch_one<28, FAM, PF, ARG>(a, ta, blocks, threads, s); break;
+    case 32: launch_one<32, FAM, PF, ARG>(a, ta, blocks, threads, s); break;
+    default: return hipErrorInvalidValue;
+  }
   return hipGetLastError();
 }
 
-template <int FAM, int PF>
-hipError_t launch_fam(int smax, const pass_args& a, int blocks, int threads, hipStream_t s,
-                      bool reduce) {
-  switch (smax) {
-    case 4: return launch_one<4, FAM, PF>(a, blocks, threads, s, reduce);
-    case 8: return launch_one<8, FAM, PF>(a, blocks, threads, s, reduce);
-    case 12: return launch_one<12, FAM, PF>(a, blocks, threads, s, reduce);
-    case 16: return launch_one<16, FAM, PF>(a, blocks, threads, s, reduce);
-    case 20: return launch_one<20, FAM, PF>(a, blocks, threads, s, reduce);
-    case 24: return launch_one<24, FAM, PF>(a, blocks, threads, s, reduce);
-    case 28: return launch_one<28, FAM, PF>(a, blocks, threads, s, reduce);
-    case 32: return launch_one<32, FAM, PF>(a, blocks, threads, s, reduce);
+template <int FAM, bool ARG>
+hipError_t launch_pass(const tile_geom& g, const pass_args& a, const theta_of<ARG>& ta,
+                       int blocks, int threads, hipStream_t s) {
+  return g.prefetch ? launch_fam<FAM, 1, ARG>(g.smax, a, ta, blocks, threads, s)
+                    : launch_fam<FAM, 0, ARG>(g.smax, a, ta, blocks, threads, s);
+}
+
+template <int FAM, bool ARG, bool HOST>
+hipError_t launch_reduce(const pass_args& a, const theta_of<ARG>& ta, int blocks, hipStream_t s) {
+  hipLaunchKernelGGL((glm_reduce_f64<FAM, ARG, HOST>), dim3(a.chains * reduce_blocks(a.K)),
+                     dim3(256), 0, s, a, blocks, ta);
+  return hipGetLastError();
+}
+
+template <int FAM>
+hipError_t launch_eval(const tile_geom& g, const pass_args& a, const double* h_theta, int blocks,
+                       int threads, hipStream_t s) {
+  hipError_t e;
+  if (a.D <= kThetaArg) {
+    theta_arg ta;
+    for (int i = 0; i < kThetaArg; ++i) ta.v[i] = i < a.D ? h_theta[i] : 0.0;
+    e = launch_pass<FAM, true>(g, a, ta, blocks, threads, s);
+    if (e == hipSuccess) e = launch_reduce<FAM, true, true>(a, ta, blocks, s);
+    return e;
   }
-  return hipErrorInvalidValue;
+  e = hipMemcpyAsync(const_cast<double*>(a.theta), h_theta, sizeof(double) * a.D,
+                     hipMemcpyHostToDevice, s);
+  if (e == hipSuccess) e = launch_pass<FAM, false>(g, a, no_theta{}, blocks, threads, s);
+  if (e == hipSuccess) e = launch_reduce<FAM, false, true>(a, no_theta{}, blocks, s);
+  return e;
 }
 
 }  // namespace
@@ -314,12 +385,20 @@ tile_geom make_geom(int64_t N, int64_t K, int L, int smax) {
 
 hipError_t launch_pass_f64(int family, const tile_geom& g, const pass_args& a,
                            int blocks, int threads, hipStream_t s, bool reduce) {
+  hipError_t e = hipErrorInvalidValue;
   if (family == SX_LOGIT)
-    return g.prefetch ? launch_fam<SX_LOGIT, 1>(g.smax, a, blocks, threads, s, reduce)
-                      : launch_fam<SX_LOGIT, 0>(g.smax, a, blocks, threads, s, reduce);
-  if (family == SX_NORMAL)
-    return g.prefetch ? launch_fam<SX_NORMAL, 1>(g.smax, a, blocks, threads, s, reduce)
-                      : launch_fam<SX_NORMAL, 0>(g.smax, a, blocks, threads, s, reduce);
+    e = launch_pass<SX_LOGIT, false>(g, a, no_theta{}, blocks, threads, s);
+  else if (family == SX_NORMAL)
+    e = launch_pass<SX_NORMAL, false>(g, a, no_theta{}, blocks, threads, s);
+  if (e != hipSuccess || !reduce) return e;
+  return family == SX_LOGIT ? launch_reduce<SX_LOGIT, false, false>(a, no_theta{}, blocks, s)
+                            : launch_reduce<SX_NORMAL, false, false>(a, no_theta{}, blocks, s);
+}
+
+hipError_t launch_eval_f64(int family, const tile_geom& g, const pass_args& a,
+                           const double* h_theta, int blocks, int threads, hipStream_t s) {
+  if (family == SX_LOGIT) return launch_eval<SX_LOGIT>(g, a, h_theta, blocks, threads, s);
+  if (family == SX_NORMAL) return launch_eval<SX_NORMAL>(g, a, h_theta, blocks, threads, s);
   return hipErrorInvalidValue;
 }
 

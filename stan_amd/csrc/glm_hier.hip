@@ -622,7 +622,7 @@ __global__ __launch_bounds__(256) void hier_mfma_x6(hier_args a) {
 // coalesced.  sum z^2 is a fixed-order shuffle reduction over the chain's
 // 32 threads.
 constexpr int kGroupsPerBlock = 8;
-template <int NR>  // entries per thread: 1 for K + 3 <= 32, else 2
+template <int NR, bool HOST>  // NR entries per thread: 1 for K + 3 <= 32, else 2
 __global__ __launch_bounds__(256) void hier_groups(hier_args a) {
   const int c = blockIdx.y * 8 + (threadIdx.x >> 5);
   const int e = threadIdx.x & 31;
@@ -688,7 +688,7 @@ __global__ __launch_bounds__(256) void hier_groups(hier_args a) {
       if (ee <= K) {
         const double tau = r == 0 ? tau0 : tau1;
         const double zv = zc[r];
-        out[1 + 2 + 2 * K + static_cast<int64_t>(g) * (K + 1) + ee] = tau * v - zv;
+        put_out<HOST>(out + 1 + 2 + 2 * K + static_cast<int64_t>(g) * (K + 1) + ee, tau * v - zv);
         szs[r] += tau * zv * v;
         zz += zv * zv;
       }
@@ -718,6 +718,7 @@ __global__ __launch_bounds__(256) void hier_groups(hier_args a) {
 // order), priors, Jacobian, output.  Every load of a slice is independent
 // and sixteen are issued before they are added, so the sums are bandwidth-
 // rather than latency-bound.
+template <bool HOST>
 __global__ __launch_bounds__(1024) void hier_final(hier_args a) {
   __shared__ double red[16][64];
   __shared__ double st[128];
@@ -771,7 +772,7 @@ __global__ __launch_bounds__(1024) void hier_final(hier_args a) {
         t = -0.5 * zz * zz + (a.propto ? 0.0 : a.alpha_const);
         ga += -th[0] / (a.alpha_sd * a.alpha_sd);
       }
-      out[1] = ga;
+      put_out<HOST>(out + 1, ga);
       lpa[0] = t;
     } else {
       const int k = ln - 1;
@@ -782,7 +783,7 @@ __global__ __launch_bounds__(1024) void hier_final(hier_args a) {
         t = -0.5 * zz * zz + (a.propto ? 0.0 : a.beta_const);
         gb += -bk / (a.beta_sd * a.beta_sd);
       }
-      out[2 + k] = gb;
+      put_out<HOST>(out + 2 + k, gb);
       lpa[ln] = t;
     }
   } else if (wv == 1 && ln <= K) {
@@ -799,7 +800,7 @@ __global__ __launch_bounds__(1024) void hier_final(hier_args a) {
       jt = v;
       gv += 1.0;
     }
-    out[2 + K + k] = gv;
+    put_out<HOST>(out + 2 + K + k, gv);
     lpt[0][k] = t;
     lpt[1][k] = jt;
   }
@@ -816,9 +817,9 @@ __global__ __launch_bounds__(1024) void hier_final(hier_args a) {
   }
   lp += -0.5 * st[2 * K + 4];
   if (!a.propto) lp += -static_cast<double>(a.J) * (K + 1) * kHalfLog2PiH;
-  out[0] = lp;
+  put_out<HOST>(out, lp);
   if (!isfinite(lp)) bad += 1.0;
-  out[a.D + 1] = bad > 0 ? 1.0 : 0.0;
+  put_out<HOST>(out + a.D + 1, bad > 0 ? 1.0 : 0.0);
 }
 
 hipError_t launch_hier_x6(const hier_args& a, dim3 grid, hipStream_t s) {
@@ -861,9 +862,22 @@ hipError_t launch_hier_mfma(const hier_args& a, dim3 grid, hipStream_t s) {
   return hipGetLastError();
 }
 
+template <bool HOST>
+hipError_t launch_hier_sums(const hier_args& a, hipStream_t s) {
+  const dim3 ggrid((a.J + kGroupsPerBlock - 1) / kGroupsPerBlock, (a.chains + 7) / 8);
+  if (a.K + 3 <= 32)
+    hipLaunchKernelGGL((hier_groups<1, HOST>), ggrid, dim3(256), 0, s, a);
+  else
+    hipLaunchKernelGGL((hier_groups<2, HOST>), ggrid, dim3(256), 0, s, a);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(hier_final<HOST>, dim3(a.chains), dim3(1024), 0, s, a);
+  return hipGetLastError();
+}
+
 }  // namespace
 
-hipError_t launch_hier(const hier_args& a, bool fp32, hipStream_t s) {
+hipError_t launch_hier(const hier_args& a, bool fp32, hipStream_t s, bool host_out) {
   if (a.K > 32 || 2 * a.K + 5 > 128 || a.chains < 1 || a.J < 1) return hipErrorInvalidValue;
   if (a.n_chunks > 0) {
     if (!fp32) {
@@ -889,15 +903,7 @@ hipError_t launch_hier(const hier_args& a, bool fp32, hipStream_t s) {
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
   }
-  const dim3 ggrid((a.J + kGroupsPerBlock - 1) / kGroupsPerBlock, (a.chains + 7) / 8);
-  if (a.K + 3 <= 32)
-    hipLaunchKernelGGL(hier_groups<1>, ggrid, dim3(256), 0, s, a);
-  else
-    hipLaunchKernelGGL(hier_groups<2>, ggrid, dim3(256), 0, s, a);
-  const hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(hier_final, dim3(a.chains), dim3(1024), 0, s, a);
-  return hipGetLastError();
+  return host_out ? launch_hier_sums<true>(a, s) : launch_hier_sums<false>(a, s);
 }
 
 }  // namespace sx

@@ -62,6 +62,13 @@ struct pass_args {
 // launch that writes out[].
 hipError_t launch_pass_f64(int family, const tile_geom& g, const pass_args& a,
                            int blocks, int threads, hipStream_t s, bool reduce = true);
+// One evaluation at a host theta: pass and reduction, with theta carried by
+// the launches where it fits (D <= kThetaArg; 3.5 KB beside pass_args in
+// the 4 KB of kernel arguments) and copied to a.theta otherwise.  a.out is
+// pinned host memory; every word of it is stored straight to the host.
+constexpr int kThetaArg = 440;
+hipError_t launch_eval_f64(int family, const tile_geom& g, const pass_args& a,
+                           const double* h_theta, int blocks, int threads, hipStream_t s);
 hipError_t launch_tile_x_f64(const double* Xrm, double* Xt, int64_t N,
                              int64_t K, const tile_geom& g, hipStream_t s);
 
@@ -113,7 +120,8 @@ struct hier_args {
   int x6;  // FP32 batches: products on BF16 MFMA in three-term splits (K <= 31)
   double alpha_sd, beta_sd, tau_sd, alpha_const, beta_const, tau_const;
 };
-hipError_t launch_hier(const hier_args& a, bool fp32, hipStream_t s);
+// host_out: a.out is pinned host memory, stored straight to the host
+hipError_t launch_hier(const hier_args& a, bool fp32, hipStream_t s, bool host_out = false);
 // 16-byte chunks of BF16 per row and term of the x6 pass's split copy of
 // X: columns 0 .. K (x' and the sign column), zero-padded to a multiple of 8
 constexpr int hier_x6_chunks(int K) { return (K + 8) / 8; }
@@ -155,8 +163,9 @@ int plain_enqueue(sx_glm* m, const double* d_theta, double* d_out, double* parti
 // the per-device scratch array of the allocation-free entry point: its
 // address on `device`, looked up once (called at context creation)
 int noalloc_setup(int device);
+int plain_eval(sx_glm* m, int propto, int jacobian);
 int hier_enqueue(sx_glm* m, hier_workspace& w, const double* d_theta, int C, double* d_out,
-                 int propto, int jacobian, bool fp32, hipStream_t stream);
+                 int propto, int jacobian, bool fp32, hipStream_t stream, bool host_out = false);
 }
 
 struct sx_glm {

@@ -1,0 +1,67 @@
+"""Single FP64 evaluations: theta carried by the launch (up to 440
+parameters) or copied, the cross-block reduction spread over blocks, and
+results stored straight to pinned host memory.  Against the FP64 oracle
+(1e-12, the plain path's bound) at the edges of each: around 440 parameters,
+one to five columns (two per wave, three waves beside the first), block
+counts around the reduction's 512-block step, and a run of calls whose
+results must not be an earlier call's."""
+import numpy as np
+import pytest
+
+import oracle as O
+import stan_amd as S
+from stan_amd import workloads as W
+
+pytestmark = pytest.mark.gpu
+TOL = 1e-12
+
+
+def _check(m, ref, th):
+    lp, g = m.log_prob_grad(th)
+    st, lp_r, g_r = ref.lpgrad(th, mode=1)
+    assert st == 0
+    assert abs(lp - lp_r) <= TOL * max(1.0, abs(lp_r))
+    assert np.linalg.norm(g - g_r) <= TOL * max(1.0, np.linalg.norm(g_r))
+
+
+@pytest.mark.parametrize("family", [S.LOGIT, S.NORMAL])
+@pytest.mark.parametrize("N,K,blocks", [(50, 1, 0), (300, 2, 0), (300, 3, 0), (64, 4, 0),
+                                        (700, 5, 0), (900, 437, 0), (900, 438, 0),
+                                        (900, 439, 0), (900, 440, 0), (40_000, 7, 511),
+                                        (140_000, 6, 513), (300_000, 3, 1024)])
+def test_eval_edges(family, N, K, blocks):
+    print(f"eval family={family} N={N} K={K} blocks={blocks}", flush=True)
+    d = W.logistic(N, K, 1.0 / np.sqrt(K), 0.5, seed=K) if family == S.LOGIT \
+        else W.normal(N, K, seed=K)
+    m = S.GlmModel(family, d["X"], d["y"], prior=d["prior"],
+                   tuning=dict(blocks=blocks, autotune=0))
+    ref = O.GlmData(family, d["X"], d["y"], prior=d["prior"])
+    for th in W.random_thetas(m.D, 3, seed=N) * 0.5:
+        _check(m, ref, th)
+    # the batched call's chains are the single evaluations
+    th = W.random_thetas(m.D, 2, seed=N + 1) * 0.5
+    lp, g = m.log_prob_grad_batch(th)
+    for c in range(2):
+        lp1, g1 = m.log_prob_grad(th[c])
+        assert lp1 == lp[c] and np.array_equal(g1, g[c])
+    m.close()
+
+
+def test_consecutive_evaluations_are_fresh():
+    """500 different points in a row, then the same in reverse."""
+    d = W.hier_logistic(J=30, K=4, seed=5, mean_log_size=np.log(30.0))
+    h = S.GlmModel(S.HIER_LOGIT, d["X"], d["y"], offsets=d["offsets"], prior=d["prior"])
+    e = W.logistic(500, 9, 0.3, 0.5, seed=2)
+    m = S.GlmModel(S.LOGIT, e["X"], e["y"], prior=e["prior"])
+    for model in (m, h):
+        ths = W.random_thetas(model.D, 500, seed=3) * 0.5
+        first = [model.log_prob_grad(t) for t in ths]
+        again = [model.log_prob_grad(t) for t in ths[::-1]][::-1]
+        assert len({lp for lp, _ in first}) == 500
+        for (la, ga), (lb, gb) in zip(first, again):
+            assert la == lb and np.array_equal(ga, gb)
+        with pytest.raises(S.DomainError):
+            model.log_prob_grad(np.full(model.D, 1e308))
+        lp, g = model.log_prob_grad(ths[0])
+        assert lp == first[0][0] and np.array_equal(g, first[0][1])
+        model.close()
