@@ -8,18 +8,14 @@
 #include <hip/hip_runtime.h>
 
 #include "sx_internal.hpp"
+#include "wave_ops.hpp"
 
 namespace sx {
 namespace {
 
 constexpr double kHalfLog2Pi = 0.91893853320467274178032973640562;
 
-// Sum of v over the 64 lanes (xor butterfly): every lane gets the total.
-__device__ __forceinline__ double wave_sum(double v) {
-#pragma unroll
-  for (int off = 1; off < 64; off <<= 1) v += __shfl_xor(v, off, 64);
-  return v;
-}
+__device__ __forceinline__ double wave_sum(double v) { return wave::sum(v); }
 
 // Stores one output value.  HOST: `p` is pinned host memory that the host
 // watches while the kernel runs, so the store goes through to it at once

@@ -175,7 +175,7 @@ __global__ __launch_bounds__(256) void glm_pass_f64(pass_args a, theta_of<ARG> t
     double e = 0.0;
 #pragma unroll
     for (int j = 0; j < SMAX; ++j) e = fma(xv[j], sb[j * L], e);
-    for (int off = 1; off < L; off <<= 1) e += __shfl_xor(e, off, 64);
+    e = wave::xor_sum(e, 1, L);
     const int64_t row = t * R + r;
     const bool valid = row < a.N;
     e += alpha;
@@ -204,11 +204,9 @@ __global__ __launch_bounds__(256) void glm_pass_f64(pass_args a, theta_of<ARG> t
   }
 
   // reduce the per-lane column partials over the R row-lanes of each column
-  for (int off = L; off < 64; off <<= 1) {
 #pragma unroll
-    for (int j = 0; j < SMAX; ++j)
-      if (j < S) acc[j] += __shfl_xor(acc[j], off, 64);
-  }
+  for (int j = 0; j < SMAX; ++j)
+    if (j < S) acc[j] = wave::xor_sum(acc[j], L, 64);
   s0 = wave_sum(s0);
   s1 = wave_sum(s1);
   bad = wave_sum(bad);
@@ -268,9 +266,9 @@ __device__ __forceinline__ void sum_entries(const double* partials, const int (&
 // one (no entry needs another's sum).  Wave 0 takes the log density (row
 // terms, residual sum, non-finite count), every other wave two columns.
 // With theta in the launches and results stored to the host, an evaluation
-// from a host theta takes 24 us at N = 3000, K = 37 (35 with one block and a
-// copy at either end), 40 us at N = 100,003, K = 129 (53) and 135 us at
-// N = 1e6, K = 100 (146, of which the pass 125).
+// from a host theta takes 22 us at N = 3000, K = 37 (35 with one block and a
+// copy at either end) and 131 us at N = 1e6, K = 100 (146), of which the
+// pass 125.
 template <int FAM, bool ARG, bool HOST>
 __global__ __launch_bounds__(256) void glm_reduce_f64(pass_args a, int nb, theta_of<ARG> ta) {
   const int per = reduce_blocks(a.K);

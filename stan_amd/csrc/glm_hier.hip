@@ -693,8 +693,11 @@ __global__ __launch_bounds__(256) void hier_groups(hier_args a) {
         zz += zv * zv;
       }
     }
-#pragma unroll
-    for (int off = 16; off > 0; off >>= 1) zz += __shfl_xor(zz, off, 32);
+    zz = wave::add_xor<16>(zz);
+    zz = wave::add_xor<8>(zz);
+    zz = wave::add_xor<4>(zz);
+    zz = wave::add_xor<2>(zz);
+    zz = wave::add_xor<1>(zz);
     szz += zz;
   }
   const int nblk = (a.J + kGroupsPerBlock - 1) / kGroupsPerBlock;

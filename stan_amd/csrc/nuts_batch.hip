@@ -30,6 +30,7 @@
 
 #include "../include/stanx/philox.hpp"
 #include "nuts_batch.hpp"
+#include "wave_ops.hpp"
 
 #pragma clang fp contract(off)
 
@@ -85,11 +86,7 @@ struct ctx {
   __device__ double* slot(int i) const { return v + static_cast<int64_t>(i) * a->Dpad; }
 };
 
-__device__ __forceinline__ double wave_sum(double x) {
-#pragma unroll
-  for (int off = 1; off < 64; off <<= 1) x += __shfl_xor(x, off, 64);
-  return x;
-}
+__device__ __forceinline__ double wave_sum(double x) { return sx::wave::sum(x); }
 // Sum of NS block totals over the chain's parts, in part order, so every
 // part gets the same values.  Wave 0 publishes this part's totals and
 // waits for every part's, one word per lane, so that the waits overlap
