@@ -36,26 +36,42 @@ constexpr double kLn2Hi = 0x1.62e42fee00000p-1;  // 32 significant bits
 constexpr double kLn2Lo = 0x1.a39ef35793c76p-33; // ln2 - kLn2Hi
 constexpr double kInvLn2 = 0x1.71547652b82fep+0;
 
+// Constants of the two series, highest order first: e^r (1/13! .. 1/0!),
+// then atanh(s)/s (1/21, 1/19 .. 1/3), then the reduction's constants.  On
+// the device they are read from constant memory, so that they arrive by
+// scalar loads and stay in scalar registers: as literals the compiler keeps
+// all of them in vector registers (46 of a lane's) across the tile loops.
+#define SX_MATH_TABLE                                                                      \
+  1.0 / 6227020800.0, 1.0 / 479001600.0, 1.0 / 39916800.0, 1.0 / 3628800.0, 1.0 / 362880.0, \
+      1.0 / 40320.0, 1.0 / 5040.0, 1.0 / 720.0, 1.0 / 120.0, 1.0 / 24.0, 1.0 / 6.0, 0.5,     \
+      1.0, 1.0, 1.0 / 21.0, 1.0 / 19.0, 1.0 / 17.0, 1.0 / 15.0, 1.0 / 13.0, 1.0 / 11.0,      \
+      1.0 / 9.0, 1.0 / 7.0, 1.0 / 5.0, 1.0 / 3.0, kInvLn2, kLn2Hi, kLn2Lo,                   \
+      0x1.a827999fcef32p-2 /* sqrt(2) - 1 */
+constexpr int kTabExp = 0, kTabLog = 14, kTabInvLn2 = 24, kTabLn2Hi = 25, kTabLn2Lo = 26,
+              kTabSqrt = 27, kTabSize = 28;
+#if defined(__HIPCC__)
+static __constant__ double sx_math_table_dev[kTabSize] = {SX_MATH_TABLE};
+#endif
+constexpr double sx_math_table[kTabSize] = {SX_MATH_TABLE};
+SX_MATH_HD double sx_tab(int i) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return sx_math_table_dev[i];
+#else
+  return sx_math_table[i];
+#endif
+}
+
 SX_MATH_HD double sx_exp_nonpos(double x) {
   if (x < -745.2) return 0.0;
-  const double k = rint(x * kInvLn2);
-  double r = fma(-k, kLn2Hi, x);
-  r = fma(-k, kLn2Lo, r);
+  const double k = rint(x * sx_tab(kTabInvLn2));
+  double r = fma(-k, sx_tab(kTabLn2Hi), x);
+  r = fma(-k, sx_tab(kTabLn2Lo), r);
   // Taylor series of e^r, Horner form, coefficients 1/n!
-  double p = 1.0 / 6227020800.0;  // 1/13!
-  p = fma(p, r, 1.0 / 479001600.0);
-  p = fma(p, r, 1.0 / 39916800.0);
-  p = fma(p, r, 1.0 / 3628800.0);
-  p = fma(p, r, 1.0 / 362880.0);
-  p = fma(p, r, 1.0 / 40320.0);
-  p = fma(p, r, 1.0 / 5040.0);
-  p = fma(p, r, 1.0 / 720.0);
-  p = fma(p, r, 1.0 / 120.0);
-  p = fma(p, r, 1.0 / 24.0);
-  p = fma(p, r, 1.0 / 6.0);
-  p = fma(p, r, 0.5);
-  p = fma(p, r, 1.0);
-  p = fma(p, r, 1.0);
+  double p = sx_tab(kTabExp);
+#if defined(__HIPCC__)
+#pragma unroll
+#endif
+  for (int i = 1; i < 14; ++i) p = fma(p, r, sx_tab(kTabExp + i));
   return ldexp(p, static_cast<int>(k));
 }
 
@@ -74,25 +90,20 @@ SX_MATH_HD double sx_rcp(double d) {
 }
 
 SX_MATH_HD double sx_log1p_unit(double t) {
-  const bool high = t > 0x1.a827999fcef32p-2;  // sqrt(2) - 1
+  const bool high = t > sx_tab(kTabSqrt);
   const double num = high ? t - 1.0 : t;        // exact (Sterbenz) when high
   const double den = high ? t + 3.0 : t + 2.0;
   const double s = num * sx_rcp(den);
   const double z = s * s;
   // atanh(s)/s = sum_k z^k / (2k + 1)
-  double p = 1.0 / 21.0;
-  p = fma(p, z, 1.0 / 19.0);
-  p = fma(p, z, 1.0 / 17.0);
-  p = fma(p, z, 1.0 / 15.0);
-  p = fma(p, z, 1.0 / 13.0);
-  p = fma(p, z, 1.0 / 11.0);
-  p = fma(p, z, 1.0 / 9.0);
-  p = fma(p, z, 1.0 / 7.0);
-  p = fma(p, z, 1.0 / 5.0);
-  p = fma(p, z, 1.0 / 3.0);
+  double p = sx_tab(kTabLog);
+#if defined(__HIPCC__)
+#pragma unroll
+#endif
+  for (int i = 1; i < 10; ++i) p = fma(p, z, sx_tab(kTabLog + i));
   const double tail = (2.0 * s) * (z * p);  // 2 atanh(s) - 2 s
   if (!high) return fma(2.0, s, tail);
-  return kLn2Hi + (fma(2.0, s, tail) + kLn2Lo);
+  return sx_tab(kTabLn2Hi) + (fma(2.0, s, tail) + sx_tab(kTabLn2Lo));
 }
 
 // Bernoulli-logit row term and residual from the linear predictor eta and
