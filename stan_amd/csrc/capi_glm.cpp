@@ -633,6 +633,7 @@ void sx_glm_destroy(sx_glm* m) {
   sx::free_workspace(m->mx);
   (void)hipFree(m->d_btheta);
   (void)hipFree(m->d_bout);
+  (void)hipFree(m->d_bpart);
   (void)hipFree(m->d_X32);
   (void)hipFree(m->d_XS);
   (void)hipFree(m->d_chunk_group);
@@ -714,6 +715,20 @@ int wait_words(sx_glm* m, const double* w, size_t n) {
   return SX_OK;
 }
 
+const char* domain_message(int family) {
+  return family == SX_LOGIT ? "bernoulli_logit_glm_lpmf: linear predictor or log density is not finite"
+         : family == SX_NORMAL
+             ? "normal_id_glm_lpdf: scale, linear predictor or log density is not finite"
+             : "bernoulli_logit_lpmf: linear predictor or log density is not finite";
+}
+
+// index of the first non-finite value, or -1
+int64_t first_non_finite(const double* x, int64_t n) {
+  for (int64_t i = 0; i < n; ++i)
+    if (!std::isfinite(x[i])) return i;
+  return -1;
+}
+
 int eval(sx_glm* m, const double* theta, int propto, int jacobian, double* lp,
          double* grad) {
   if (!m || !theta || !lp) {
@@ -722,11 +737,10 @@ int eval(sx_glm* m, const double* theta, int propto, int jacobian, double* lp,
   }
   SX_HIP(hipSetDevice(m->device));
   const size_t D = static_cast<size_t>(m->D);
-  for (size_t i = 0; i < D; ++i)
-    if (!std::isfinite(theta[i])) {
-      set_error("log_prob: parameter " + std::to_string(i) + " is not finite");
-      return SX_EDOMAIN;
-    }
+  if (const int64_t bad = first_non_finite(theta, m->D); bad >= 0) {
+    set_error("log_prob: parameter " + std::to_string(bad) + " is not finite");
+    return SX_EDOMAIN;
+  }
   std::memcpy(m->h_theta, theta, D * sizeof(double));
   int rc;
   if (m->family == SX_HIER_LOGIT) {
@@ -750,10 +764,7 @@ int eval(sx_glm* m, const double* theta, int propto, int jacobian, double* lp,
   *lp = m->h_out[0];
   if (grad) std::memcpy(grad, m->h_out + 1, D * sizeof(double));
   if (m->h_out[D + 1] != 0.0) {
-    set_error(m->family == SX_LOGIT ? "bernoulli_logit_glm_lpmf: linear predictor or log density is not finite"
-              : m->family == SX_NORMAL
-                  ? "normal_id_glm_lpdf: scale, linear predictor or log density is not finite"
-                  : "bernoulli_logit_lpmf: linear predictor or log density is not finite");
+    set_error(domain_message(m->family));
     return SX_EDOMAIN;
   }
   return SX_OK;
@@ -815,12 +826,15 @@ static pass_args plain_args(const sx_glm* m, const double* theta, double* out, d
   return a;
 }
 
-// The FP64 pass of a logistic or normal context: theta (device, D) ->
-// out (device, D + 2), per-block partials in `partials` (blocks x (K + 3)
-// doubles), on `stream`.
+// The FP64 pass of a logistic or normal context: theta (device, chains x D)
+// -> out (device, chains x (D + 2)), per-block partials in `partials`
+// (chains x blocks x (K + 3) doubles), on `stream`.
 int plain_enqueue(sx_glm* m, const double* d_theta, double* d_out, double* partials, int propto,
-                  int jacobian, hipStream_t stream, bool reduce) {
-  const pass_args a = plain_args(m, d_theta, d_out, partials, propto, jacobian);
+                  int jacobian, hipStream_t stream, bool reduce, int chains) {
+  pass_args a = plain_args(m, d_theta, d_out, partials, propto, jacobian);
+  a.chains = chains;
+  a.theta_stride = m->D;
+  a.out_stride = m->D + 2;
   SX_HIP(launch_pass_f64(m->family, m->geom, a, m->blocks, m->threads, stream, reduce));
   return SX_OK;
 }
@@ -1092,6 +1106,57 @@ int ensure_batch_staging(sx_glm* m, int64_t C) {
   return SX_OK;
 }
 
+// C chains of a logistic or normal context in FP64, evaluated together in
+// slabs whose block partials stay within kSlabBytes.  Each chain's result is
+// bitwise its single evaluation's.  A chain at a non-finite theta, or with a
+// non-finite density, gets lp = -inf and the call reports SX_EDOMAIN; at a
+// non-finite theta its gradient is left as it was.
+constexpr size_t kSlabBytes = size_t(256) << 20;
+
+int fp64_batch(sx_glm* m, const double* theta, int64_t C, int propto, int jacobian, double* lp,
+               double* grad) {
+  SX_HIP(hipSetDevice(m->device));
+  const int64_t D = m->D, E = m->K + 3;
+  const int64_t fit = static_cast<int64_t>(kSlabBytes / (sizeof(double) * E * m->blocks));
+  const int64_t slab = std::max<int64_t>(1, std::min<int64_t>({C, fit, 1024}));
+  int rc = ensure_batch_staging(m, slab);
+  if (rc) return rc;
+  if (m->bpart_cap < slab) {
+    (void)hipFree(m->d_bpart);
+    m->d_bpart = nullptr;
+    m->bpart_cap = 0;
+    SX_HIP(hipMalloc(&m->d_bpart, sizeof(double) * E * m->blocks * slab));
+    m->bpart_cap = slab;
+  }
+  std::vector<double> out(static_cast<size_t>(slab * (D + 2)));
+  int worst = SX_OK;
+  for (int64_t b = 0; b < C; b += slab) {
+    const int64_t n = std::min(slab, C - b);
+    const double* th = theta + b * D;
+    SX_HIP(hipMemcpyAsync(m->d_btheta, th, sizeof(double) * n * D, hipMemcpyHostToDevice,
+                          m->stream));
+    rc = sx::plain_enqueue(m, m->d_btheta, m->d_bout, m->d_bpart, propto, jacobian, m->stream,
+                           true, static_cast<int>(n));
+    if (rc) return rc;
+    SX_HIP(hipMemcpyAsync(out.data(), m->d_bout, sizeof(double) * n * (D + 2),
+                          hipMemcpyDeviceToHost, m->stream));
+    SX_HIP(hipStreamSynchronize(m->stream));
+    for (int64_t c = 0; c < n; ++c) {
+      const int64_t bad = first_non_finite(th + c * D, D);
+      const double* o = out.data() + c * (D + 2);
+      lp[b + c] = o[0];
+      if (bad < 0 && grad) std::memcpy(grad + (b + c) * D, o + 1, sizeof(double) * D);
+      if (bad >= 0 || o[D + 1] != 0.0) {
+        lp[b + c] = -INFINITY;
+        worst = SX_EDOMAIN;
+        set_error(bad >= 0 ? "log_prob: parameter " + std::to_string(bad) + " is not finite"
+                           : domain_message(m->family));
+      }
+    }
+  }
+  return worst;
+}
+
 }  // namespace
 
 extern "C" {
@@ -1144,18 +1209,10 @@ int sx_glm_logp_grad_batch(sx_glm* m, const double* theta, int64_t C, int propto
     }
     return worst;
   }
-  int worst = SX_OK;
-  for (int64_t c = 0; c < C; ++c) {
-    int rc = eval(m, theta + c * m->D, propto, jacobian, lp + c,
-                  grad ? grad + c * m->D : nullptr);
-    if (rc == SX_EDOMAIN) {
-      lp[c] = -INFINITY;
-      worst = SX_EDOMAIN;
-    } else if (rc) {
-      return rc;
-    }
-  }
-  return worst;
+  if (C > 1) return fp64_batch(m, theta, C, propto, jacobian, lp, grad);
+  const int rc = eval(m, theta, propto, jacobian, lp, grad);
+  if (rc == SX_EDOMAIN) lp[0] = -INFINITY;
+  return rc;
 }
 
 int sx_glm_time_logp_grad(sx_glm* m, const double* theta, int64_t C, int iters, int warmup,

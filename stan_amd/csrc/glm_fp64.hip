@@ -8,7 +8,7 @@
 //             SS = sum d_n^2, r_n = d_n
 // and the adjoint X^T r, sum r, reading every element of X exactly once:
 // each wave loads a 64-row-block tile of X into registers (one 512-byte
-// coalesced load per slot), forms eta with an L-lane shuffle reduction,
+// coalesced load per slot), forms eta with an L-lane reduction,
 // evaluates the link, and accumulates x * r into per-lane FP64 registers.
 // Block partials are summed in a fixed order by a second one-block launch,
 // so results are bitwise reproducible, and that launch adds the priors and
@@ -23,24 +23,12 @@
 
 #include "../include/stanx/sx_math.hpp"
 #include "glm_finalize.hpp"
+#include "glm_fp64_tile.hpp"
 #include "sx_internal.hpp"
 
 namespace sx {
 
 namespace {
-
-// Buffer-resource loads: lanes whose offset is past `bytes` read zero and
-// generate no memory request, so a tile's SMAX slot loads need no
-// branches when the layout only holds S <= SMAX slots.
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* base,
-                                                            uint32_t bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), static_cast<short>(0),
-                                           static_cast<int>(bytes), 0x00020000);
-}
-__device__ __forceinline__ double buf_f64(__amdgpu_buffer_rsrc_t r, uint32_t voff,
-                                          uint32_t soff) {
-  return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, voff, soff, 2));
-}
 
 // Blocks of the cross-block reduction per chain: four waves each, wave 0
 // for the log density, the others two columns.
@@ -53,23 +41,6 @@ __device__ __forceinline__ void load_tile(const pass_args& a, int64_t t, int lan
       make_rsrc(a.X + t * static_cast<int64_t>(a.S) * 64, static_cast<uint32_t>(a.S) * 512u);
 #pragma unroll
   for (int j = 0; j < SMAX; ++j) x[j] = buf_f64(rs, lane * 8u, j * 512u);
-}
-
-// y of this lane's row (zero past N); issued before the tile's X loads so
-// that waiting for it leaves the X loads in flight
-template <int FAM>
-__device__ __forceinline__ double load_y(const pass_args& a, int64_t t, int R, int r) {
-  const int64_t row0 = t * R;
-  const int64_t rows = a.N - row0 < R ? a.N - row0 : R;
-  if (FAM == SX_LOGIT) {
-    const __amdgpu_buffer_rsrc_t rs =
-        make_rsrc(static_cast<const int8_t*>(a.y) + row0, static_cast<uint32_t>(rows));
-    return static_cast<double>(__builtin_amdgcn_raw_buffer_load_b8(rs, r, 0, 0));
-  } else {
-    const __amdgpu_buffer_rsrc_t rs =
-        make_rsrc(static_cast<const double*>(a.y) + row0, static_cast<uint32_t>(rows) * 8u);
-    return buf_f64(rs, r * 8u, 0);
-  }
 }
 
 // A single evaluation's theta travels in the kernel arguments (ARG; D <=
@@ -123,9 +94,9 @@ __global__ __launch_bounds__(256) void glm_pass_f64(pass_args a, theta_of<ARG> t
   const int wib = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int nw = blockDim.x >> 6;
   const int L = a.L;
-  const int q = lane & (L - 1);
-  const int r = lane >> a.lgL;
   const int R = 64 >> a.lgL;
+  const int q = lane >> (6 - a.lgL);
+  const int r = lane & (R - 1);
   const int S = a.S;
 
   // the first tile's loads are issued before theta is staged: the two
@@ -175,7 +146,7 @@ __global__ __launch_bounds__(256) void glm_pass_f64(pass_args a, theta_of<ARG> t
     double e = 0.0;
 #pragma unroll
     for (int j = 0; j < SMAX; ++j) e = fma(xv[j], sb[j * L], e);
-    e = wave::xor_sum(e, 1, L);
+    e = wave::xor_sum(e, R, 64);
     const int64_t row = t * R + r;
     const bool valid = row < a.N;
     e += alpha;
@@ -204,9 +175,7 @@ __global__ __launch_bounds__(256) void glm_pass_f64(pass_args a, theta_of<ARG> t
   }
 
   // reduce the per-lane column partials over the R row-lanes of each column
-#pragma unroll
-  for (int j = 0; j < SMAX; ++j)
-    if (j < S) acc[j] = wave::xor_sum(acc[j], L, 64);
+  wave::xor_sum_n<SMAX>(acc, 1, R);
   s0 = wave_sum(s0);
   s1 = wave_sum(s1);
   bad = wave_sum(bad);
@@ -304,8 +273,9 @@ __global__ void tile_x_f64(const double* __restrict__ Xrm, double* __restrict__ 
   const int64_t js = idx >> 6;  // t * S + j
   const int64_t t = js / S;
   const int j = static_cast<int>(js - t * S);
-  const int64_t row = t * (64 >> lgL) + (lane >> lgL);
-  const int64_t col = static_cast<int64_t>(j) * L + (lane & (L - 1));
+  const int lgR = 6 - lgL;
+  const int64_t row = (t << lgR) + (lane & ((1 << lgR) - 1));
+  const int64_t col = static_cast<int64_t>(j) * L + (lane >> lgR);
   Xt[idx] = (row < N && col < K) ? Xrm[row * K + col] : 0.0;
 }
 
@@ -338,6 +308,8 @@ hipError_t launch_fam(int smax, const pass_args& a, const theta_of<ARG>& ta, int
 template <int FAM, bool ARG>
 hipError_t launch_pass(const tile_geom& g, const pass_args& a, const theta_of<ARG>& ta,
                        int blocks, int threads, hipStream_t s) {
+  if constexpr (!ARG)
+    if (chains_pass_fits(g, a, threads)) return launch_pass_f64_chains(FAM, g, a, blocks, s);
   return g.prefetch ? launch_fam<FAM, 1, ARG>(g.smax, a, ta, blocks, threads, s)
                     : launch_fam<FAM, 0, ARG>(g.smax, a, ta, blocks, threads, s);
 }

@@ -62,6 +62,23 @@ struct pass_args {
 // launch that writes out[].
 hipError_t launch_pass_f64(int family, const tile_geom& g, const pass_args& a,
                            int blocks, int threads, hipStream_t s, bool reduce = true);
+// The bulk pass of several chains that share tiles of X (glm_fp64_chains.hip):
+// the same partials, bit for bit, as the single-chain pass.
+hipError_t launch_pass_f64_chains(int family, const tile_geom& g, const pass_args& a, int blocks,
+                                  hipStream_t s);
+// Whether a batch takes it.  It needs L <= 4 lanes per row (a DPP row of 16
+// lanes then holds rows of one column group), a wave's worth of chains for
+// each of its four waves, and work to outweigh its longer latency.  Measured
+// us, single-chain pass over a grid of chains -> this one: N = 1e6, K = 100,
+// 32 chains 2678 -> 848, 8 chains 741 -> 365; N = 200,003, K = 60, 32 chains
+// 281 -> 137; around the line N = 20,000, K = 20, 32 chains 24.9 -> 23.7, N =
+// 50,000, K = 20, 8 chains 18.7 -> 18.3; below it N = 10,000, K = 50, 8
+// chains 13.0 -> 19.5, N = 3000, K = 37, 32 chains 11.1 -> 17.0.
+inline bool chains_pass_fits(const tile_geom& g, const pass_args& a, int threads) {
+  return a.chains >= 8 && threads == 256 && g.L <= 4 && g.S > 0 &&
+         a.N * a.K * a.chains >= (int64_t(1) << 23);
+}
+
 // One evaluation at a host theta: pass and reduction, with theta carried by
 // the launches where it fits (D <= kThetaArg; 3.5 KB beside pass_args in
 // the 4 KB of kernel arguments) and copied to a.theta otherwise.  a.out is
@@ -159,7 +176,7 @@ int mx_enqueue(sx_glm* m, mx_workspace& w, const double* d_theta, int C, double*
 int hier_prepare(sx_glm* m, hier_workspace& w, int C);
 int mx_autotune(sx_glm* m);
 int plain_enqueue(sx_glm* m, const double* d_theta, double* d_out, double* partials, int propto,
-                  int jacobian, hipStream_t stream, bool reduce);
+                  int jacobian, hipStream_t stream, bool reduce, int chains = 1);
 // the per-device scratch array of the allocation-free entry point: its
 // address on `device`, looked up once (called at context creation)
 int noalloc_setup(int device);
@@ -193,6 +210,8 @@ struct sx_glm {
   double* d_btheta = nullptr;  // batched theta / out staging for the C-ABI batch call
   double* d_bout = nullptr;
   int64_t bcap = 0;
+  double* d_bpart = nullptr;  // block partials of the FP64 batch call
+  int64_t bpart_cap = 0;      // chains
   // hierarchical model
   float* d_X32 = nullptr;
   uint16_t* d_XS = nullptr;  // split copy of the sign-folded X (FP32, K <= 31)

@@ -65,3 +65,54 @@ def test_consecutive_evaluations_are_fresh():
         lp, g = model.log_prob_grad(ths[0])
         assert lp == first[0][0] and np.array_equal(g, first[0][1])
         model.close()
+
+
+@pytest.mark.parametrize("family", [S.LOGIT, S.NORMAL])
+@pytest.mark.parametrize("N,K,L,cap,blocks,C", [
+    (120_011, 9, 1, 12, 384, 8), (70_001, 13, 1, 16, 300, 11), (50_000, 32, 1, 32, 77, 9),
+    (64_033, 17, 2, 12, 256, 8), (61_007, 37, 2, 20, 513, 17), (300_001, 3, 2, 4, 2048, 10),
+    (60_005, 60, 4, 16, 512, 8), (33_333, 63, 4, 16, 1024, 13), (30_001, 101, 4, 28, 255, 8),
+    (21_000, 128, 4, 32, 512, 16), (66_000, 29, 4, 8, 64, 33)])
+def test_chains_pass_is_the_single_pass(family, N, K, L, cap, blocks, C):
+    """Batches large enough for the several-chains pass: every chain bitwise
+    its single evaluation, over its forms (1, 2 and 4 lanes per row; slots
+    odd, even and full; X values held and read again; one tile per sequence,
+    odd and even tile counts; a partial last tile; block counts that do and do
+    not divide by 8; a last group of 1, 2, 3 or 8 chains), and the first
+    against the oracle (1e-12)."""
+    print(f"chains family={family} N={N} K={K} L={L} blocks={blocks} C={C}", flush=True)
+    assert N * K * C >= 1 << 23
+    d = W.logistic(N, K, 1.0 / np.sqrt(K), 0.5, seed=K) if family == S.LOGIT \
+        else W.normal(N, K, seed=K)
+    m = S.GlmModel(family, d["X"], d["y"], prior=d["prior"],
+                   tuning=dict(lanes_per_row=L, slots_cap=cap, blocks=blocks, autotune=0))
+    th = W.random_thetas(m.D, C, seed=N) * 0.5
+    th[3, 1] = 1e308  # eta overflows: this chain alone has no density
+    lp, g = m.log_prob_grad_batch(th)
+    assert np.isneginf(lp[3])
+    for c in range(C):
+        if c == 3:
+            continue
+        lp1, g1 = m.log_prob_grad(th[c])
+        assert lp1 == lp[c], c
+        assert np.array_equal(g1, g[c]), c
+    ref = O.GlmData(family, d["X"], d["y"], prior=d["prior"])
+    st, lp_r, g_r = ref.lpgrad(th[0], mode=1)
+    assert abs(lp[0] - lp_r) <= TOL * abs(lp_r)
+    assert np.linalg.norm(g[0] - g_r) <= TOL * np.linalg.norm(g_r)
+    m.close()
+
+
+def test_batch_of_a_non_finite_point():
+    """A chain at a non-finite theta: -inf, its gradient row left alone, the
+    others unaffected."""
+    d = W.normal(900, 5, seed=3)
+    m = S.GlmModel(S.NORMAL, d["X"], d["y"], prior=d["prior"])
+    th = W.random_thetas(m.D, 3, seed=1) * 0.3
+    th[1, 2] = np.nan
+    lp, g = m.log_prob_grad_batch(th)
+    assert np.isneginf(lp[1]) and np.all(g[1] == 0.0)
+    for c in (0, 2):
+        lp1, g1 = m.log_prob_grad(th[c])
+        assert lp1 == lp[c] and np.array_equal(g1, g[c])
+    m.close()
