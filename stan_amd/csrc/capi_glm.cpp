@@ -14,6 +14,7 @@
 #include <mutex>
 #include <sstream>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "sx_internal.hpp"
@@ -642,6 +643,7 @@ void sx_glm_destroy(sx_glm* m) {
   sx::free_workspace(m->hw);
   if (m->h_theta) (void)hipHostFree(m->h_theta);
   if (m->h_out) (void)hipHostFree(m->h_out);
+  if (m->h_batch) (void)hipHostFree(m->h_batch);
   if (m->ev0) (void)hipEventDestroy(m->ev0);
   if (m->ev1) (void)hipEventDestroy(m->ev1);
   if (m->stream) (void)hipStreamDestroy(m->stream);
@@ -722,10 +724,18 @@ const char* domain_message(int family) {
              : "bernoulli_logit_lpmf: linear predictor or log density is not finite";
 }
 
-// index of the first non-finite value, or -1
+// index of the first non-finite value, or -1 (blocks are checked without an
+// early exit, which the compiler vectorises)
 int64_t first_non_finite(const double* x, int64_t n) {
-  for (int64_t i = 0; i < n; ++i)
-    if (!std::isfinite(x[i])) return i;
+  constexpr int64_t kBlock = 256;
+  for (int64_t b = 0; b < n; b += kBlock) {
+    const int64_t e = std::min(n, b + kBlock);
+    int bad = 0;
+    for (int64_t i = b; i < e; ++i) bad |= !(std::fabs(x[i]) <= 1.7976931348623157e308);
+    if (bad)
+      for (int64_t i = b; i < e; ++i)
+        if (!std::isfinite(x[i])) return i;
+  }
   return -1;
 }
 
@@ -1106,21 +1116,120 @@ int ensure_batch_staging(sx_glm* m, int64_t C) {
   return SX_OK;
 }
 
+// largest batch the pinned buffer holds, in bytes
+constexpr size_t kPinnedBytes = size_t(64) << 20;
+
+// Pinned buffer of the batch calls, kept by the context.  One for both ways:
+// a batch's results are copied into it only after its points have left it
+// (stream order), and pinning costs about 0.1 ms per MB at the first call.
+int ensure_batch_pinned(sx_glm* m, int64_t C) {
+  if (m->hbcap >= C) return SX_OK;
+  if (m->h_batch) (void)hipHostFree(m->h_batch);
+  m->h_batch = nullptr;
+  m->hbcap = 0;
+  SX_HIP(hipHostMalloc(&m->h_batch, sizeof(double) * C * (m->D + 2)));
+  m->hbcap = C;
+  return SX_OK;
+}
+
+// fn(0) .. fn(n - 1) on up to four threads when `bytes` of copying are worth
+// them (a thread starts in about 15 us, a core copies about 10 KB/us)
+template <class F>
+void spread_rows(int64_t n, size_t bytes, F fn) {
+  const int64_t nt = std::min<int64_t>({n, 4, static_cast<int64_t>(bytes >> 20)});
+  std::vector<std::thread> th;
+  int64_t done = 0;  // rows that threads have taken
+  try {
+    for (int64_t i = 0; i + 1 < nt; ++i) {
+      const int64_t a = n * i / nt, b = n * (i + 1) / nt;
+      th.emplace_back([=] {
+        for (int64_t r = a; r < b; ++r) fn(r);
+      });
+      done = b;
+    }
+  } catch (...) {  // no more threads: this one takes the rest
+  }
+  for (int64_t r = done; r < n; ++r) fn(r);
+  for (auto& t : th) t.join();
+}
+
+// Runs a batched evaluation of C chains in slabs of at most `slab`: points to
+// the device, enqueue(n) for the kernels (d_btheta -> d_bout), results back
+// to lp and grad.  checked: a chain at a non-finite theta is a domain error
+// whose gradient is left as it was.  A chain with a domain error gets lp =
+// -inf and the call reports SX_EDOMAIN.
+//
+// The host copies bound a large batch (64 x 21,042 parameters, 10.8 MB each
+// way: 1670 us per call through the runtime's staging of pageable memory,
+// 1060 through a pinned buffer filled and emptied by four threads, of which
+// the kernels 88).  Small batches take the pinned buffer too (15 KB: 163 ->
+// 155 us).  Between kSmallBytes and kLargeBytes a single thread reads what a
+// copy engine has just written more slowly than the runtime's staging
+// delivers it (528 KB: 302 us pageable, 307 pinned).
+constexpr size_t kSmallBytes = size_t(64) << 10, kLargeBytes = size_t(1) << 20;
+
+template <class F>
+int batch_call(sx_glm* m, const double* theta, int64_t C, int64_t slab, bool checked,
+               const char* message, double* lp, double* grad, F enqueue) {
+  SX_HIP(hipSetDevice(m->device));
+  const int64_t D = m->D;
+  const size_t row = sizeof(double) * static_cast<size_t>(D);
+  slab = std::max<int64_t>(
+      1, std::min<int64_t>({C, slab, static_cast<int64_t>(kPinnedBytes / (row + 16))}));
+  const size_t most = slab * (row + 16);
+  const bool pinned = most < kSmallBytes || most >= kLargeBytes;
+  int rc = ensure_batch_staging(m, slab);
+  if (rc == SX_OK && pinned) rc = ensure_batch_pinned(m, slab);
+  if (rc) return rc;
+  if (!pinned && m->bout.size() < most / sizeof(double)) m->bout.resize(most / sizeof(double));
+  const double* const out = pinned ? m->h_batch : m->bout.data();
+  int worst = SX_OK;
+  for (int64_t b = 0; b < C; b += slab) {
+    const int64_t n = std::min(slab, C - b);
+    const double* th = theta + b * D;
+    const double* src = th;
+    if (pinned) {
+      spread_rows(n, n * row,
+                  [=](int64_t c) { std::memcpy(m->h_batch + c * D, th + c * D, row); });
+      src = m->h_batch;
+    }
+    SX_HIP(hipMemcpyAsync(m->d_btheta, src, n * row, hipMemcpyHostToDevice, m->stream));
+    rc = enqueue(static_cast<int>(n));
+    if (rc) return rc;
+    SX_HIP(hipMemcpyAsync(const_cast<double*>(out), m->d_bout, n * (row + 16),
+                          hipMemcpyDeviceToHost, m->stream));
+    SX_HIP(hipStreamSynchronize(m->stream));
+    for (int64_t c = 0; c < n; ++c) {
+      const int64_t bad = checked ? first_non_finite(th + c * D, D) : -1;
+      const double* o = out + c * (D + 2);
+      lp[b + c] = o[0];
+      if (bad >= 0 || o[D + 1] != 0.0) {
+        lp[b + c] = -INFINITY;
+        worst = SX_EDOMAIN;
+        set_error(bad >= 0 ? "log_prob: parameter " + std::to_string(bad) + " is not finite"
+                           : std::string(message));
+      }
+    }
+    if (grad)
+      spread_rows(n, n * row, [=](int64_t c) {
+        if (!checked || first_non_finite(th + c * D, D) < 0)
+          std::memcpy(grad + (b + c) * D, out + c * (D + 2) + 1, row);
+      });
+  }
+  return worst;
+}
+
 // C chains of a logistic or normal context in FP64, evaluated together in
 // slabs whose block partials stay within kSlabBytes.  Each chain's result is
-// bitwise its single evaluation's.  A chain at a non-finite theta, or with a
-// non-finite density, gets lp = -inf and the call reports SX_EDOMAIN; at a
-// non-finite theta its gradient is left as it was.
+// bitwise its single evaluation's.
 constexpr size_t kSlabBytes = size_t(256) << 20;
 
 int fp64_batch(sx_glm* m, const double* theta, int64_t C, int propto, int jacobian, double* lp,
                double* grad) {
   SX_HIP(hipSetDevice(m->device));
-  const int64_t D = m->D, E = m->K + 3;
+  const int64_t E = m->K + 3;
   const int64_t fit = static_cast<int64_t>(kSlabBytes / (sizeof(double) * E * m->blocks));
   const int64_t slab = std::max<int64_t>(1, std::min<int64_t>({C, fit, 1024}));
-  int rc = ensure_batch_staging(m, slab);
-  if (rc) return rc;
   if (m->bpart_cap < slab) {
     (void)hipFree(m->d_bpart);
     m->d_bpart = nullptr;
@@ -1128,33 +1237,11 @@ int fp64_batch(sx_glm* m, const double* theta, int64_t C, int propto, int jacobi
     SX_HIP(hipMalloc(&m->d_bpart, sizeof(double) * E * m->blocks * slab));
     m->bpart_cap = slab;
   }
-  std::vector<double> out(static_cast<size_t>(slab * (D + 2)));
-  int worst = SX_OK;
-  for (int64_t b = 0; b < C; b += slab) {
-    const int64_t n = std::min(slab, C - b);
-    const double* th = theta + b * D;
-    SX_HIP(hipMemcpyAsync(m->d_btheta, th, sizeof(double) * n * D, hipMemcpyHostToDevice,
-                          m->stream));
-    rc = sx::plain_enqueue(m, m->d_btheta, m->d_bout, m->d_bpart, propto, jacobian, m->stream,
-                           true, static_cast<int>(n));
-    if (rc) return rc;
-    SX_HIP(hipMemcpyAsync(out.data(), m->d_bout, sizeof(double) * n * (D + 2),
-                          hipMemcpyDeviceToHost, m->stream));
-    SX_HIP(hipStreamSynchronize(m->stream));
-    for (int64_t c = 0; c < n; ++c) {
-      const int64_t bad = first_non_finite(th + c * D, D);
-      const double* o = out.data() + c * (D + 2);
-      lp[b + c] = o[0];
-      if (bad < 0 && grad) std::memcpy(grad + (b + c) * D, o + 1, sizeof(double) * D);
-      if (bad >= 0 || o[D + 1] != 0.0) {
-        lp[b + c] = -INFINITY;
-        worst = SX_EDOMAIN;
-        set_error(bad >= 0 ? "log_prob: parameter " + std::to_string(bad) + " is not finite"
-                           : domain_message(m->family));
-      }
-    }
-  }
-  return worst;
+  return batch_call(m, theta, C, slab, true, domain_message(m->family), lp, grad,
+                    [=](int n) {
+    return sx::plain_enqueue(m, m->d_btheta, m->d_bout, m->d_bpart, propto, jacobian, m->stream,
+                             true, n);
+  });
 }
 
 }  // namespace
@@ -1178,36 +1265,16 @@ int sx_glm_logp_grad_batch(sx_glm* m, const double* theta, int64_t C, int propto
   }
   if (C == 0) return SX_OK;
   if (m->precision == SX_BF16X2 || m->family == SX_HIER_LOGIT) {
-    SX_HIP(hipSetDevice(m->device));
-    int rc = ensure_batch_staging(m, C);
-    if (rc) return rc;
-    const int64_t D = m->D;
-    SX_HIP(hipMemcpyAsync(m->d_btheta, theta, sizeof(double) * C * D, hipMemcpyHostToDevice,
-                          m->stream));
-    rc = m->family == SX_HIER_LOGIT
-             ? sx::hier_enqueue(m, m->hw, m->d_btheta, static_cast<int>(C), m->d_bout, propto,
-                                jacobian, m->precision == SX_FP32, m->stream)
-             : sx::mx_enqueue(m, m->mx, m->d_btheta, static_cast<int>(C), m->d_bout, propto,
-                              jacobian, m->stream);
-    if (rc) return rc;
-    std::vector<double> out(static_cast<size_t>(C * (D + 2)));
-    SX_HIP(hipMemcpyAsync(out.data(), m->d_bout, sizeof(double) * out.size(),
-                          hipMemcpyDeviceToHost, m->stream));
-    SX_HIP(hipStreamSynchronize(m->stream));
-    int worst = SX_OK;
-    for (int64_t c = 0; c < C; ++c) {
-      const double* o = out.data() + c * (D + 2);
-      lp[c] = o[0];
-      if (grad) std::memcpy(grad + c * D, o + 1, sizeof(double) * D);
-      if (o[D + 1] != 0.0) {
-        lp[c] = -INFINITY;
-        worst = SX_EDOMAIN;
-        set_error(m->family == SX_HIER_LOGIT
-                      ? "bernoulli_logit_lpmf: linear predictor or log density is not finite"
-                      : "batched GLM: linear predictor or log density is not finite");
-      }
-    }
-    return worst;
+    const bool hier = m->family == SX_HIER_LOGIT;
+    return batch_call(m, theta, C, C, false,
+                      hier ? domain_message(m->family)
+                           : "batched GLM: linear predictor or log density is not finite",
+                      lp, grad, [=](int n) {
+                        return hier ? sx::hier_enqueue(m, m->hw, m->d_btheta, n, m->d_bout, propto,
+                                                       jacobian, m->precision == SX_FP32, m->stream)
+                                    : sx::mx_enqueue(m, m->mx, m->d_btheta, n, m->d_bout, propto,
+                                                     jacobian, m->stream);
+                      });
   }
   if (C > 1) return fp64_batch(m, theta, C, propto, jacobian, lp, grad);
   const int rc = eval(m, theta, propto, jacobian, lp, grad);

@@ -116,3 +116,19 @@ def test_batch_of_a_non_finite_point():
         lp1, g1 = m.log_prob_grad(th[c])
         assert lp1 == lp[c] and np.array_equal(g1, g[c])
     m.close()
+
+
+@pytest.mark.parametrize("J,C", [(3, 5), (60, 40), (60, 300), (3000, 140)])
+def test_batch_staging_sizes(J, C):
+    """Batches whose points go through the pinned buffer (small, and large on
+    several threads), around it (between 64 KB and 1 MB), and in two slabs
+    (70 MB): chains bitwise their single evaluations."""
+    d = W.hier_logistic(J=J, K=20, seed=J, mean_log_size=np.log(4.0))
+    m = S.GlmModel(S.HIER_LOGIT, d["X"], d["y"], offsets=d["offsets"], prior=d["prior"])
+    th = W.random_thetas(m.D, C, seed=C) * 0.3
+    print(f"staging J={J} C={C}: {th.nbytes} bytes", flush=True)
+    lp, g = m.log_prob_grad_batch(th)
+    for c in sorted({0, 1, C // 2, C - 9 if C > 9 else 0, C - 1}):
+        lp1, g1 = m.log_prob_grad(th[c])
+        assert lp1 == lp[c] and np.array_equal(g1, g[c]), c
+    m.close()
