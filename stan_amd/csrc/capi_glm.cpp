@@ -867,16 +867,21 @@ int mx_chain_pad(const sx_glm* m, int C) {
   return (C + 127) / 128 * 128;
 }
 
+// row splits for a target of tps tiles each: a multiple of 8, at most 512
+static int mx_splits(const sx_glm* m, int64_t tps) {
+  const int64_t n_tiles = m->Np / 32;
+  if (tps <= 0) tps = 8;
+  return static_cast<int>(
+      std::min<int64_t>(512, std::max<int64_t>(8, ((n_tiles + tps - 1) / tps + 7) / 8 * 8)));
+}
+
 int mx_prepare(sx_glm* m, mx_workspace& w, int C) {
   if (!m->d_Xh) {
     set_error("batched BF16 evaluation needs a context created with SX_BF16X2");
     return SX_EINVAL;
   }
   const int Cp = mx_chain_pad(m, C);
-  const int64_t n_tiles = m->Np / 32;
-  const int64_t tps = m->mx_tps > 0 ? m->mx_tps : 8;
-  int splits = static_cast<int>(
-      std::min<int64_t>(512, std::max<int64_t>(8, ((n_tiles + tps - 1) / tps + 7) / 8 * 8)));
+  const int splits = mx_splits(m, m->mx_tps);
   if (w.cap >= Cp && w.splits == splits) return SX_OK;
   free_workspace(w);
   const size_t ck = static_cast<size_t>(Cp) * m->Kp;
@@ -950,9 +955,9 @@ int mx_enqueue(sx_glm* m, mx_workspace& w, const double* d_theta, int C, double*
 // waves split by k where Kp / 32 is even and at most 8; or, for Kp <= 128,
 // one wave per block without operand prefetch at two waves per SIMD, the
 // same products as the first) and the row split
-// (target tiles of 32 rows per split: 4 to 128; at most 512 splits, so
-// large N reach fewer splits, and fewer gradient partials to sum, only with
-// the larger targets), each timed as full
+// (target tiles of 32 rows per split; at most 512 splits, so large N reach
+// fewer splits, and fewer gradient partials to sum, only with the larger
+// targets), each timed as full
 // evaluations of 128 chains at theta = 0 (the kernels' work does not depend
 // on the values).  The split sets the order of the FP64 sums, so, as for
 // the FP64 pass, the first decision per (device, family, N, K) is kept for
@@ -989,10 +994,28 @@ int mx_autotune(sx_glm* m) {
   const int kq = static_cast<int>(m->Kp / 32);
   int best_v = 0, best_t = 8;
   double best_ms = 1e30;
+  // Targets: 4 to 128 tiles per split, and those that give half, one and two
+  // splits per CU, so that the workgroups of one or two chain blocks fill
+  // whole rounds of the device (N = 2e5, K = 256: 200 splits make 400
+  // workgroups for 256 chains, 1.6 rounds of 256 CUs; 256 splits make two).
+  // Each split count is timed once.
+  int cus = 0;
+  if (rc == SX_OK) rc = device_cus(&cus);
+  const int64_t n_tiles = m->Np / 32;
+  std::vector<int> targets, seen;
+  for (int64_t t : {int64_t(4), int64_t(8), int64_t(16), int64_t(32), int64_t(64), int64_t(128),
+                    (2 * n_tiles + cus - 1) / std::max(1, cus), (n_tiles + cus - 1) / std::max(1, cus),
+                    (n_tiles + 2 * cus - 1) / std::max(1, 2 * cus)}) {
+    t = std::max<int64_t>(1, t);
+    const int sp = mx_splits(m, t);
+    if (std::find(seen.begin(), seen.end(), sp) != seen.end()) continue;
+    seen.push_back(sp);
+    targets.push_back(static_cast<int>(t));
+  }
   for (int v = 0; v <= 2 && rc == SX_OK; ++v) {
     if (v == 1 && (m->Kp > 256 || kq % 2 != 0)) continue;
     if (v == 2 && kq > 4) continue;
-    for (int tps : {4, 8, 16, 32, 64, 128}) {
+    for (int tps : targets) {
       m->mx_variant = v;
       m->mx_tps = tps;
       for (int i = 0; i < 2 && rc == SX_OK; ++i)
