@@ -574,7 +574,7 @@ __global__ __launch_bounds__(128 * NCB) void glm_mfma32_pair(mx_args a) {
 // operands the adjoint will use, lane by lane (tile t, 32-chain group g,
 // half st: the lane's bf16x8 at R[((t * Cp / 32 + g) * 2 + st) * 64 +
 // lane]), and the row terms per split.  glm_mfma32_adj then forms
-// G^T = R^T X per block of 256 k.
+// G^T = R^T X per block of 128 k.
 template <int KQ, int FAM, int NW>
 __global__ __launch_bounds__(64 * NW) void glm_mfma32_fwd(mx_args a) {
   static_assert(KQ > 8 && KQ <= 16 && KQ % 2 == 0, "glm_mfma32_fwd handles 256 < Kp <= 512, Kp % 64 == 0");
@@ -716,11 +716,16 @@ __global__ __launch_bounds__(64 * NW) void glm_mfma32_fwd(mx_args a) {
 // columns from column 32 kq0): G^T (32 chains x 32 k) += R^T X per tile,
 // as in glm_mfma32 (step st takes the lane's residuals of rows 8 (j/4) +
 // 4 h + j%4, j = 8 st .. 8 st + 7, and the same rows of X through the
-// transposing LDS read), with R read from the forward launch's output and
-// the tile's column block of X staged through LDS one tile ahead.
+// transposing LDS read), with R read from the forward launch's output one
+// tile ahead and the tile's column block of X staged through LDS likewise.
+// One launch covers all column blocks (128 columns each, a last one of 64
+// where Kp / 64 is odd), a workgroup per row split, chain block and column
+// block: with 64 chains the splits alone are fewer workgroups than the chip
+// has CUs (N = 48,176, K = 468: two launches of 256 columns 2 x 21.6 us, one
+// of 128 columns 22.8 us).
 template <int KQA, int NW>
-__global__ __launch_bounds__(64 * NW) void glm_mfma32_adj(mx_args a, int kq0) {
-  static_assert(KQA >= 1 && KQA <= 8, "blocks of at most 256 columns");
+__device__ __forceinline__ void adj_block(const mx_args& a, int kq0, int spl, int cblk,
+                                          __bf16* xa, __bf16* xb) {
   static_assert((4 * KQA) % NW == 0, "staging blocks per wave");
   constexpr int KR = 32 * KQA;         // columns of the block
   constexpr int CPRB = KR / 8;         // 16-byte chunks per block row
@@ -728,17 +733,10 @@ __global__ __launch_bounds__(64 * NW) void glm_mfma32_adj(mx_args a, int kq0) {
   constexpr int TE = 32 * KR;          // elements of one tile array
   constexpr int BPA = 2 * KQA;         // 1 KB staging blocks per tile array
   constexpr int NBW = 2 * BPA / NW;
-  __shared__ __attribute__((aligned(16))) __bf16 xa[2 * TE];
-  __shared__ __attribute__((aligned(16))) __bf16 xb[2 * TE];
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int li = lane & 31, h = lane >> 5;
-  const int nCB = a.Cp / (32 * NW);
-  const int bid = blockIdx.x;
-  const int xcd = bid & 7, widx = bid >> 3;
-  const int spl = (widx / nCB) * 8 + xcd;
-  const int cblk = widx % nCB;
   const int cbase = cblk * 32 * NW + 32 * w;
   const int64_t g32 = cbase / 32, nG = a.Cp / 32;
   const int Kp = a.Kp;
@@ -768,19 +766,27 @@ __global__ __launch_bounds__(64 * NW) void glm_mfma32_adj(mx_args a, int kq0) {
           (lds_ptr)((XB) + (b_ / BPA) * TE + bb_ * 512), 16, 0, 0);              \
     }                                                                            \
   }
+  bf16x8 rh[2], rl[2], nrh[2], nrl[2];
+  auto load_r = [&](int64_t t) {
+#pragma unroll
+    for (int st = 0; st < 2; ++st) {
+      const int64_t ri = ((t * nG + g32) * 2 + st) * 64 + lane;
+      nrh[st] = Rh[ri];
+      nrl[st] = Rl[ri];
+    }
+  };
   auto tile = [&](const __bf16* X, int64_t t) {
+#pragma unroll
+    for (int st = 0; st < 2; ++st) {
+      rh[st] = nrh[st];
+      rl[st] = nrl[st];
+    }
+    if (t + 1 < t1) load_r(t + 1);
     int ln = lane;
     asm volatile("" : "+v"(ln));
     const tile_addr<2 * KR, P> ad(ln);
     const char* xb = reinterpret_cast<const char*>(X);
     constexpr int TB = 64 * KR;
-    bf16x8 rh[2], rl[2];
-#pragma unroll
-    for (int st = 0; st < 2; ++st) {
-      const int64_t ri = ((t * nG + g32) * 2 + st) * 64 + lane;
-      rh[st] = Rh[ri];
-      rl[st] = Rl[ri];
-    }
 #pragma unroll
     for (int st = 0; st < 2; ++st) {
 #pragma unroll
@@ -793,7 +799,10 @@ __global__ __launch_bounds__(64 * NW) void glm_mfma32_adj(mx_args a, int kq0) {
       }
     }
   };
-  if (t0 < t1) SX_STAGE(t0, xa);
+  if (t0 < t1) {
+    SX_STAGE(t0, xa);
+    load_r(t0);
+  }
   __builtin_amdgcn_s_waitcnt(0);
   __syncthreads();
   for (int64_t t = t0; t < t1; t += 2) {
@@ -818,29 +827,54 @@ __global__ __launch_bounds__(64 * NW) void glm_mfma32_adj(mx_args a, int kq0) {
     }
 }
 
+// grid: splits x chain blocks x column blocks, the workgroups of one split 8
+// block ids apart (one XCD: they share the split's residuals in its L2)
+template <int NW>
+__global__ __launch_bounds__(64 * NW) void glm_mfma32_adj(mx_args a) {
+  constexpr int TE = 32 * 128;
+  __shared__ __attribute__((aligned(16))) __bf16 xa[2 * TE];
+  __shared__ __attribute__((aligned(16))) __bf16 xb[2 * TE];
+  const int nCB = a.Cp / (32 * NW), nK = (a.Kp + 127) / 128;
+  const int bid = blockIdx.x;
+  const int xcd = bid & 7, widx = bid >> 3;
+  const int cblk = widx % nCB;
+  const int kb = widx / nCB % nK;
+  const int spl = widx / (nCB * nK) * 8 + xcd;
+  if (4 * kb + 4 <= a.Kp / 32)
+    adj_block<4, NW>(a, 4 * kb, spl, cblk, xa, xb);
+  else
+    adj_block<2, NW>(a, 4 * kb, spl, cblk, xa, xb);
+}
+
 // Per chain: FP64 sums of the split partials, then priors and output.  A
-// split's gradient partials are a contiguous row of Kp floats; the block's
-// 1024 threads cover the rows as Kp/4 float4 columns x 4096/Kp slices of
-// splits, every thread active and eight 16-byte loads in flight.  Each
-// thread sums its splits in ascending order, the slices are combined in
-// slice order: a fixed order that depends on N, K and the split count only.
-template <int FAM>
-__global__ __launch_bounds__(1024) void mx_reduce(mx_args a, pass_args pa) {
-  extern __shared__ double st[];
-  __shared__ double red[4096];  // [slice][k], Kp x slices = 4096
+// split's gradient partials are a contiguous row of Kp floats, covered as Kp /
+// 4 float4 columns x nsl = 4096 / Kp slices of splits; RB blocks per chain
+// take 1 / RB of the columns each (no column needs another's sum), the first
+// also the row terms, the log density and the status.  Each thread
+// sums its splits in ascending order with eight 16-byte loads in flight, the
+// slices are combined in slice order: a fixed order that depends on N, K and
+// the split count only.  RB = 4 up to 64 chains, where one block per chain
+// leaves most CUs idle (64 chains, 192 splits, K = 468: 11.2 us with RB = 1,
+// 9.1 with 4); more chains fill the chip, and whole rows read better (256
+// chains, 512 splits, K = 100: 16.6 us with RB = 1, 19.4 with 4).
+template <int FAM, int RB>
+__global__ __launch_bounds__(1024 / RB) void mx_reduce(mx_args a, pass_args pa) {
+  __shared__ double red[4096 / RB];  // [slice][column of the block]
   __shared__ double rs[3][64];
-  const int c = blockIdx.x;
-  pa.theta += static_cast<int64_t>(c) * pa.theta_stride;
-  pa.out += static_cast<int64_t>(c) * pa.out_stride;
+  const int c = static_cast<int>(blockIdx.x) / RB;
+  const int part = static_cast<int>(blockIdx.x) % RB;
+  const double* theta = pa.theta + static_cast<int64_t>(c) * pa.theta_stride;
+  double* out = pa.out + static_cast<int64_t>(c) * pa.out_stride;
   const int K = pa.K, Kp = a.Kp;
-  const int q = Kp / 4;               // float4 columns of a row
-  const int nsl = 1024 / q;           // slices of splits (q * nsl <= 1024)
+  const int nsl = 1024 / (Kp / 4);    // slices of splits
+  const int q = Kp / 4 / RB;          // float4 columns of the block (q * nsl <= 1024 / RB)
   const int tid = threadIdx.x;
   const int kq = tid % q, sl = tid / q;
+  const int k0 = 4 * q * part;        // first column of the block
   const int64_t gstride = static_cast<int64_t>(a.Cp) * Kp;
-  const float* gp = a.gpart + static_cast<int64_t>(c) * Kp + 4 * kq;
+  const float* gp = a.gpart + static_cast<int64_t>(c) * Kp + k0 + 4 * kq;
   double v[4] = {0, 0, 0, 0};
-  // threads past q * nsl (Kp not dividing 4096) take no splits
+  // threads past q * nsl take no splits
   int si = sl < nsl ? sl : a.splits;
   for (; si + 7 * nsl < a.splits; si += 8 * nsl) {
     float4 x[8];
@@ -864,10 +898,10 @@ __global__ __launch_bounds__(1024) void mx_reduce(mx_args a, pass_args pa) {
   }
   if (sl < nsl)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) red[sl * Kp + 4 * kq + i] = v[i];
+    for (int i = 0; i < 4; ++i) red[sl * (4 * q) + 4 * kq + i] = v[i];
   // row terms (lp, sum r, bad): entry e on threads 64 e .. 64 e + 63, each
   // over splits l, l + 64, ... (eight loads in flight), then the 64 in order
-  if (tid < 192) {
+  if (part == 0 && tid < 192) {
     const int e = tid >> 6, l = tid & 63;
     const double* sp = a.spart + static_cast<int64_t>(c) * 3 + e;
     const int64_t sstride = 3 * static_cast<int64_t>(a.Cp);
@@ -884,18 +918,22 @@ __global__ __launch_bounds__(1024) void mx_reduce(mx_args a, pass_args pa) {
     rs[e][l] = t;
   }
   __syncthreads();
-  if (tid < K) {
+  if (tid < 4 * q && k0 + tid < K) {
     double t = 0.0;
-    for (int s2 = 0; s2 < nsl; ++s2) t += red[s2 * Kp + tid];
-    st[2 + tid] = t;  // finalize layout: st[0] lp, st[1] sum r, st[2 + k], st[K + 2] bad
-  } else if (tid >= 1021) {
-    const int e = tid - 1021;
-    double t = 0.0;
-    for (int l = 0; l < 64; ++l) t += rs[e][l];
-    st[e == 0 ? 0 : (e == 1 ? 1 : K + 2)] = t;
+#pragma unroll 8
+    for (int s2 = 0; s2 < nsl; ++s2) t += red[s2 * (4 * q) + tid];
+    finalize_beta<FAM, false>(pa, theta, out, k0 + tid, t);
   }
-  __syncthreads();
-  if (tid < 64) finalize<FAM>(pa, st);
+  // the last wave adds the row terms, on lanes 0 .. 2
+  constexpr int T0 = 1024 / RB - 64;
+  if (part == 0 && tid >= T0) {
+    const int e = tid - T0 < 3 ? tid - T0 : 0;
+    double t = 0.0;
+#pragma unroll 8
+    for (int l = 0; l < 64; ++l) t += rs[e][l];
+    finalize_head<FAM, false>(pa, theta, out, __shfl(t, 0, 64), __shfl(t, 1, 64),
+                              __shfl(t, 2, 64));
+  }
 }
 
 template <int KQ, int NW, bool PF = true>
@@ -941,7 +979,7 @@ hipError_t launch_kq32(int family, const mx_args& a, hipStream_t s) {
   return launch_kq32_nw<KQ, 4>(family, a, s);
 }
 
-// 256 < Kp <= 512: forward + link, then the adjoint per block of 256 k
+// 256 < Kp <= 512: forward + link, then the adjoint of all column blocks
 template <int KQ, int NW>
 hipError_t launch_wide_nw(int family, const mx_args& a, hipStream_t s) {
   if (a.splits % 8 != 0 || a.Cp % (32 * NW) != 0 || !a.Rh || !a.Rl) return hipErrorInvalidValue;
@@ -952,10 +990,8 @@ hipError_t launch_wide_nw(int family, const mx_args& a, hipStream_t s) {
     hipLaunchKernelGGL((glm_mfma32_fwd<KQ, SX_NORMAL, NW>), grid, dim3(64 * NW), 0, s, a);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL((glm_mfma32_adj<8, NW>), grid, dim3(64 * NW), 0, s, a, 0);
-  e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  hipLaunchKernelGGL((glm_mfma32_adj<KQ - 8, NW>), grid, dim3(64 * NW), 0, s, a, 8);
+  hipLaunchKernelGGL((glm_mfma32_adj<NW>), dim3(grid.x * ((a.Kp + 127) / 128)), dim3(64 * NW), 0, s,
+                     a);
   return hipGetLastError();
 }
 template <int KQ>
@@ -1013,11 +1049,15 @@ hipError_t launch_mfma_pass(int family, const double* theta, int64_t D, int C, c
     default: return hipErrorInvalidValue;
   }
   if (e != hipSuccess) return e;
-  const size_t lds = static_cast<size_t>(pa.E) * sizeof(double);
-  if (family == SX_LOGIT)
-    hipLaunchKernelGGL((mx_reduce<SX_LOGIT>), dim3(C), dim3(1024), lds, s, a, pa);
+  const bool few = C <= 64;
+  if (family == SX_LOGIT && few)
+    hipLaunchKernelGGL((mx_reduce<SX_LOGIT, 4>), dim3(C * 4), dim3(256), 0, s, a, pa);
+  else if (family == SX_LOGIT)
+    hipLaunchKernelGGL((mx_reduce<SX_LOGIT, 1>), dim3(C), dim3(1024), 0, s, a, pa);
+  else if (few)
+    hipLaunchKernelGGL((mx_reduce<SX_NORMAL, 4>), dim3(C * 4), dim3(256), 0, s, a, pa);
   else
-    hipLaunchKernelGGL((mx_reduce<SX_NORMAL>), dim3(C), dim3(1024), lds, s, a, pa);
+    hipLaunchKernelGGL((mx_reduce<SX_NORMAL, 1>), dim3(C), dim3(1024), 0, s, a, pa);
   return hipGetLastError();
 }
 

@@ -103,15 +103,6 @@ __device__ __forceinline__ void finalize_head(const pass_args& a, const double* 
   put_out<HOST>(out + a.D + 1, bad > 0 ? 1.0 : 0.0);
 }
 
-// Both, from the reduced statistics in LDS: writes out[0] = lp, out[1..D] =
-// gradient, out[D+1] = status (0 ok, 1 domain error).  Runs on one wave.
-template <int FAM>
-__device__ void finalize(const pass_args& a, const double* st) {
-  for (int k = threadIdx.x & 63; k < a.K; k += 64)
-    finalize_beta<FAM, false>(a, a.theta, a.out, k, st[2 + k]);
-  finalize_head<FAM, false>(a, a.theta, a.out, st[0], st[1], st[a.K + 2]);
-}
-
 }  // namespace
 }  // namespace sx
 #endif
