@@ -173,16 +173,28 @@ int create_batch(sx_nuts_batch** out, sx_glm* m, const sx_nuts_config* cfg, int6
     }
     b->a.parts = parts;
     b->a.spin_limit = 1 << 22;
-    // Phase turns per chain and launch: above 8192 coordinates a chain's
-    // vector passes cost about as much as its gradient, and one chain
-    // closing a deep subtree (a merge pass per level, then the transition)
-    // would hold the whole step; such a chain yields after 4 turns and
-    // continues in the next step.  Below, a yield's extra step (a batched
-    // gradient) costs more than the wait.  Measured totals (ms/step x
-    // steps): hierarchical D = 21,042, 64 chains: 1008 unbounded, 954
-    // with 6, 908 with 4, 950 with 3; logistic D = 101, 256 chains: 2508
-    // unbounded, 2807 with 4.  STANX_NUTS_PHASE_BUDGET=n sets it (n >= 1).
-    b->a.phase_budget = D > 8192 ? 4 : 4096;
+    // Phase turns per chain and launch.  One chain closing a deep subtree
+    // (a merge pass per level, then the transition) holds the whole step;
+    // with a bound such a chain yields after 4 turns and continues in the
+    // next step, whose batched gradient is the price.  Draws and gradients
+    // are the same either way.  Bounded where the waits cost more than the
+    // extra gradients:
+    //  - above 8192 coordinates always (a vector pass costs about as much
+    //    as the gradient).  Hierarchical D = 21,042, 64 chains, ms in all:
+    //    1008 unbounded, 954 with 6, 908 with 4, 950 with 3;
+    //  - below, for gradients under about 50 us (N K chains <= 2^30,
+    //    FP32 / BF16) and enough work per step for one chain to stand out
+    //    (D >= 32, D chains >= 2048).  ms unbounded / with 4: logistic
+    //    20000 x 100, 256 chains 164 / 149; x 200 239 / 208; 64 chains
+    //    127 / 119; hierarchical FP32, 64 chains, D = 612 74 / 63,
+    //    D = 1812 105 / 82, D = 7722 149 / 122.
+    // On the other side of those lines: 1e6 x 100, 24 chains 271 / 286;
+    // hierarchical 2^30.6 123 / 127; D = 11, 16 chains 21.3 / 24.2;
+    // D = 104, 16 chains 41.6 / 42.7; FP64 40000 x 50, 32 chains
+    // 132 / 135.  STANX_NUTS_PHASE_BUDGET=n sets it (n >= 1).
+    const bool cheap = grad_precision != SX_FP64 && D >= 32 && D * chains >= 2048 &&
+                       static_cast<double>(m->N) * m->K * chains <= 1073741824.0;
+    b->a.phase_budget = D > 8192 || cheap ? 4 : 4096;
     if (const char* e = std::getenv("STANX_NUTS_PHASE_BUDGET"))
       b->a.phase_budget = std::max(1, std::atoi(e));
     if (parts > 1) {
