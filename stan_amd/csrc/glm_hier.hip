@@ -615,67 +615,44 @@ __global__ __launch_bounds__(256) void hier_mfma_x6(hier_args a) {
 // Per group and chain: sum the group's chunks in order; z gradients;
 // per-group contributions [S_0..S_K, z.S terms (K+1), lp, bad, sum z^2],
 // summed over the block's groups in group order: the block's row of
-// partials, [(chain x blocks + block) x G].  A block takes kGroupsPerBlock
-// consecutive groups and 8 chains (32 threads per chain; tau = exp(v)
-// computed once per chain and block): a chunk's partials of those chains
-// are contiguous (chain-major, E entries each), so the block reads them
-// coalesced.  sum z^2 is a fixed-order shuffle reduction over the chain's
-// 32 threads.
+// partials, [(chain x blocks + block) x G].  Latency-bound (offsets, then
+// partials, then the sums): a block takes kGroupsPerBlock consecutive
+// groups of one chain side by side, TW threads each, and adds their totals
+// from LDS.  The chains of a block of groups are neighbours on one XCD
+// (grid x: chain, block mod 8; y, z: block / 8), where rows of
+// E entries share cache lines.  sum z^2 is a fixed-order lane sum.  us, a
+// block walking its groups one after the other with 8 chains in it, and
+// this: J = 1000, K = 20, ~3500 chunks: 1 chain 13.2 / 5.0, 8 chains
+// 12.5 / 6.4, 64 chains 23.2 / 21.1; J = 100 1 chain 13.1 / 4.7.
 constexpr int kGroupsPerBlock = 8;
-template <int NR, bool HOST>  // NR entries per thread: 1 for K + 3 <= 32, else 2
-__global__ __launch_bounds__(256) void hier_groups(hier_args a) {
-  const int c = blockIdx.y * 8 + (threadIdx.x >> 5);
-  const int e = threadIdx.x & 31;
-  if (c >= a.chains) return;  // a whole 32-thread chain group
+template <int TW, int NR, bool HOST>  // TW x NR >= K + 3 entries
+__global__ __launch_bounds__(8 * TW) void hier_groups(hier_args a) {
+  constexpr int kW = TW * NR;
+  // per group: [S_e x kW, tau z x kW, sum z^2]
+  __shared__ double gsum[kGroupsPerBlock][2 * kW + 1];
+  const int nblk = (a.J + kGroupsPerBlock - 1) / kGroupsPerBlock;
+  const int c = blockIdx.x >> 3;
+  const int blk = (blockIdx.z * gridDim.y + blockIdx.y) * 8 + (blockIdx.x & 7);
+  if (blk >= nblk) return;
+  const int e = threadIdx.x % TW, q = threadIdx.x / TW;
   const int K = a.K;
   const double* th = a.theta + static_cast<int64_t>(c) * a.theta_stride;
   double* out = a.out + static_cast<int64_t>(c) * a.out_stride;
-  // entries e and e + 32 (K <= 32: at most two per thread)
-  const double tau0 = e <= K ? exp(th[1 + K + e]) : 0.0;
-  const double tau1 = NR > 1 && e + 32 <= K ? exp(th[1 + K + e + 32]) : 0.0;
-  const int g0 = blockIdx.x * kGroupsPerBlock;
-  const int g1 = g0 + kGroupsPerBlock < a.J ? g0 + kGroupsPerBlock : a.J;
-  double sv[NR], szs[NR], szz = 0.0;  // sums over the block's groups
-#pragma unroll
-  for (int r = 0; r < NR; ++r) sv[r] = szs[r] = 0.0;
-  // the first (up to) eight chunk partials and the z entries of a group,
-  // loaded one group ahead so that the next group's loads are in flight
-  // while this one is summed
-  double xn[NR][8], zn[NR];
-  auto load_head = [&](int g) {
-    const int64_t c0 = a.group_chunk0[g], c1 = a.group_chunk0[g + 1];
-    const double* z = th + 2 + 2 * K + static_cast<int64_t>(g) * (K + 1);
-#pragma unroll
-    for (int r = 0; r < NR; ++r) {
-      const int ee = e + 32 * r;
-#pragma unroll
-      for (int u = 0; u < 8; ++u)
-        xn[r][u] = (ee < K + 3 && c0 + u < c1) ? a.cpart[((c0 + u) * a.chains + c) * a.E + ee] : 0.0;
-      zn[r] = ee <= K ? z[ee] : 0.0;
-    }
-  };
-  if (g0 < g1) load_head(g0);
-  for (int g = g0; g < g1; ++g) {
+  const int g0 = blk * kGroupsPerBlock;
+  const int ng = a.J - g0 < kGroupsPerBlock ? a.J - g0 : kGroupsPerBlock;
+  if (q < ng) {  // all TW threads of a group
+    const int g = g0 + q;
     const int64_t ch0 = a.group_chunk0[g], ch1 = a.group_chunk0[g + 1];
-    double xc[NR][8], zc[NR];
-#pragma unroll
-    for (int r = 0; r < NR; ++r) {
-      zc[r] = zn[r];
-#pragma unroll
-      for (int u = 0; u < 8; ++u) xc[r][u] = xn[r][u];
-    }
-    if (g + 1 < g1) load_head(g + 1);
+    const double* z = th + 2 + 2 * K + static_cast<int64_t>(g) * (K + 1);
     double zz = 0.0;
 #pragma unroll
     for (int r = 0; r < NR; ++r) {
-      const int ee = e + 32 * r;
+      const int ee = e + TW * r;
       if (ee >= K + 3) continue;
-      // chunks in order: the preloaded head, then eight loads in flight
+      const double tau = ee <= K ? exp(th[1 + K + ee]) : 0.0;
+      const double zv = ee <= K ? z[ee] : 0.0;
       double v = 0.0;
-#pragma unroll
-      for (int u = 0; u < 8; ++u)
-        if (ch0 + u < ch1) v += xc[r][u];
-      int64_t ch = ch0 + 8;
+      int64_t ch = ch0;
       for (; ch + 8 <= ch1; ch += 8) {
         double x[8];
 #pragma unroll
@@ -683,37 +660,52 @@ __global__ __launch_bounds__(256) void hier_groups(hier_args a) {
 #pragma unroll
         for (int u = 0; u < 8; ++u) v += x[u];
       }
-      for (; ch < ch1; ++ch) v += a.cpart[(ch * a.chains + c) * a.E + ee];
-      sv[r] += v;
+      double x[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+        x[u] = ch + u < ch1 ? a.cpart[((ch + u) * a.chains + c) * a.E + ee] : 0.0;
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+        if (ch + u < ch1) v += x[u];
+      gsum[q][ee] = v;
       if (ee <= K) {
-        const double tau = r == 0 ? tau0 : tau1;
-        const double zv = zc[r];
         put_out<HOST>(out + 1 + 2 + 2 * K + static_cast<int64_t>(g) * (K + 1) + ee, tau * v - zv);
-        szs[r] += tau * zv * v;
+        gsum[q][kW + ee] = tau * zv;
         zz += zv * zv;
       }
     }
-    zz = wave::add_xor<16>(zz);
+    if (TW > 16) zz = wave::add_xor<16>(zz);
     zz = wave::add_xor<8>(zz);
     zz = wave::add_xor<4>(zz);
     zz = wave::add_xor<2>(zz);
     zz = wave::add_xor<1>(zz);
-    szz += zz;
+    if (e == 0) gsum[q][2 * kW] = zz;
   }
-  const int nblk = (a.J + kGroupsPerBlock - 1) / kGroupsPerBlock;
-  double* gs = a.gpart + (static_cast<int64_t>(c) * nblk + blockIdx.x) * a.G;
+  __syncthreads();
+  if (q != 0) return;
+  double* gs = a.gpart + (static_cast<int64_t>(c) * nblk + blk) * a.G;
 #pragma unroll
   for (int r = 0; r < NR; ++r) {
-    const int ee = e + 32 * r;
+    const int ee = e + TW * r;
     if (ee >= K + 3) continue;
+    double sv = 0.0, szs = 0.0;
+    for (int i = 0; i < ng; ++i) {
+      const double v = gsum[i][ee];
+      sv += v;
+      if (ee <= K) szs += gsum[i][kW + ee] * v;
+    }
     if (ee <= K) {
-      gs[ee] = sv[r];
-      gs[K + 1 + ee] = szs[r];
+      gs[ee] = sv;
+      gs[K + 1 + ee] = szs;
     } else {
-      gs[K + 1 + ee] = sv[r];  // lp (ee = K+1) at 2K+2, bad (ee = K+2) at 2K+3
+      gs[K + 1 + ee] = sv;  // lp (ee = K+1) at 2K+2, bad (ee = K+2) at 2K+3
     }
   }
-  if (e == 0) gs[2 * K + 4] = szz;
+  if (e == 0) {
+    double szz = 0.0;
+    for (int i = 0; i < ng; ++i) szz += gsum[i][2 * kW];
+    gs[2 * K + 4] = szz;
+  }
 }
 
 // Per chain: sums over the group blocks' rows (sixteen fixed interleaved
@@ -867,11 +859,15 @@ hipError_t launch_hier_mfma(const hier_args& a, dim3 grid, hipStream_t s) {
 
 template <bool HOST>
 hipError_t launch_hier_sums(const hier_args& a, hipStream_t s) {
-  const dim3 ggrid((a.J + kGroupsPerBlock - 1) / kGroupsPerBlock, (a.chains + 7) / 8);
-  if (a.K + 3 <= 32)
-    hipLaunchKernelGGL((hier_groups<1, HOST>), ggrid, dim3(256), 0, s, a);
+  const int nb8 = ((a.J + kGroupsPerBlock - 1) / kGroupsPerBlock + 7) / 8;
+  const int ny = nb8 < 32768 ? nb8 : 32768;
+  const dim3 grid(8 * a.chains, ny, (nb8 + ny - 1) / ny);
+  if (a.K + 3 <= 16)
+    hipLaunchKernelGGL((hier_groups<16, 1, HOST>), grid, dim3(128), 0, s, a);
+  else if (a.K + 3 <= 32)
+    hipLaunchKernelGGL((hier_groups<32, 1, HOST>), grid, dim3(256), 0, s, a);
   else
-    hipLaunchKernelGGL((hier_groups<2, HOST>), ggrid, dim3(256), 0, s, a);
+    hipLaunchKernelGGL((hier_groups<32, 2, HOST>), grid, dim3(256), 0, s, a);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(hier_final<HOST>, dim3(a.chains), dim3(1024), 0, s, a);
