@@ -15,6 +15,7 @@
 #include <sstream>
 #include <string>
 #include <thread>
+#include <utility>
 #include <vector>
 
 #include "sx_internal.hpp"
@@ -226,6 +227,8 @@ int hier_chunks(sx_glm* m, const int64_t* off, int chunk) {
   (void)hipFree(m->d_chunk_group);
   (void)hipFree(m->d_chunk_row0);
   (void)hipFree(m->d_group_chunk0);
+  (void)hipFree(m->d_by_rows);
+  m->d_by_rows = nullptr;
   m->d_chunk_group = nullptr;
   m->d_chunk_row0 = m->d_group_chunk0 = nullptr;
   m->n_chunks = static_cast<int64_t>(cg.size());
@@ -237,6 +240,22 @@ int hier_chunks(sx_glm* m, const int64_t* off, int chunk) {
     SX_HIP(hipMemcpy(m->d_chunk_group, cg.data(), sizeof(int) * cg.size(), hipMemcpyHostToDevice));
   SX_HIP(hipMemcpy(m->d_chunk_row0, cr0.data(), sizeof(int64_t) * cr0.size(), hipMemcpyHostToDevice));
   SX_HIP(hipMemcpy(m->d_group_chunk0, gc0.data(), sizeof(int64_t) * gc0.size(), hipMemcpyHostToDevice));
+  if (m->precision == SX_FP32 && !cg.empty()) {
+    // most rows first, by a counting sort over the rows (1 .. chunk)
+    std::vector<int64_t> at(static_cast<size_t>(chunk) + 1, 0);
+    const auto rows = [&](size_t i) {  // a group's last chunk ends with the group
+      return static_cast<int>(std::min<int64_t>(off[cg[i] + 1] - cr0[i], chunk));
+    };
+    for (size_t i = 0; i < cg.size(); ++i) ++at[chunk - rows(i)];
+    int64_t sum = 0;
+    for (int64_t& v : at) sum += std::exchange(v, sum);
+    std::vector<sx::hier_chunk> t(cg.size());
+    for (size_t i = 0; i < cg.size(); ++i)
+      t[at[chunk - rows(i)]++] = {cr0[i], rows(i), cg[i], static_cast<int>(i), 0};
+    SX_HIP(hipMalloc(&m->d_by_rows, sizeof(sx::hier_chunk) * t.size()));
+    SX_HIP(hipMemcpy(m->d_by_rows, t.data(), sizeof(sx::hier_chunk) * t.size(),
+                     hipMemcpyHostToDevice));
+  }
   return SX_OK;
 }
 
@@ -640,6 +659,7 @@ void sx_glm_destroy(sx_glm* m) {
   (void)hipFree(m->d_chunk_group);
   (void)hipFree(m->d_chunk_row0);
   (void)hipFree(m->d_group_chunk0);
+  (void)hipFree(m->d_by_rows);
   sx::free_workspace(m->hw);
   if (m->h_theta) (void)hipHostFree(m->h_theta);
   if (m->h_out) (void)hipHostFree(m->h_out);
@@ -1099,6 +1119,8 @@ int hier_enqueue(sx_glm* m, hier_workspace& w, const double* d_theta, int C, dou
   a.chunk_group = m->d_chunk_group;
   a.chunk_row0 = m->d_chunk_row0;
   a.group_chunk0 = m->d_group_chunk0;
+  a.by_rows = m->d_by_rows;
+  a.simds = m->max_blocks / 2;
   a.n_chunks = m->n_chunks;
   a.theta_stride = m->D;
   a.out_stride = m->D + 2;

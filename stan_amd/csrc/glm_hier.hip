@@ -160,8 +160,8 @@ __global__ __launch_bounds__(256) void hier_pass_f64(hier_args a) {
 #undef SX_LOAD_BLOCK
 }
 
-// FP32 on the matrix cores: a wave per chunk and up to 64 chains (NH
-// halves of 32).  X is stored sign-folded, x' = s x with s = 2y - 1, and
+// FP32 on the matrix cores: a wave per chunk and 32 NH chains.  X is
+// stored sign-folded, x' = s x with s = 2y - 1, and
 // each staged row carries s itself as column K, so one product per tile
 // and half gives the base-2 margin of every (row, chain):
 //   q = log2(e) s eta = sum_k x'_k w'_k + s b',  w' = log2(e) w, b' = log2(e) b
@@ -202,12 +202,20 @@ __global__ __launch_bounds__(256) void hier_mfma_f32(hier_args a) {
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int li = lane & 31, h = lane >> 5;
-  const int64_t ch = static_cast<int64_t>(blockIdx.x) * 4 + w;
-  if (ch >= a.n_chunks) return;  // whole wave; no block barrier follows
-  const int g = a.chunk_group[ch];
-  const int64_t r0 = a.chunk_row0[ch], r1 = a.chunk_row0[ch + 1];
-  const int rows = static_cast<int>(r1 - r0);
-  const int cb = blockIdx.y * (32 * NH);
+  // the wave's item: rounds of one wave per SIMD take the chunks from the
+  // longest to the shortest, every other round from its end, so that the
+  // SIMDs' shares are even.  With ragged groups the busiest SIMD had twice
+  // the mean's tiles in data order: J = 1000 of ~100 rows (sd of the log
+  // 1), K = 10, 64 chains: 32.1 -> 20.8 us (matrix cores alone ~8).
+  const unsigned ncb = (a.chains + 32 * NH - 1) / (32 * NH);
+  const unsigned round = blockIdx.z * gridDim.y + blockIdx.y;
+  const unsigned in = blockIdx.x * 4 + w;
+  const unsigned item = round * a.simds + ((round & 1) ? a.simds - 1 - in : in);
+  if (item >= a.n_chunks * ncb) return;  // whole wave; no block barrier follows
+  const hier_chunk hc = a.by_rows[item / ncb];
+  const int64_t ch = hc.id, r0 = hc.row0;
+  const int g = hc.group, rows = hc.rows;
+  const int cb = static_cast<int>(item % ncb) * (32 * NH);
   // chain coefficients: half hf, chain cb + 32 hf + i, column 2 s + h
   float wk[NH][NJ];
 #pragma unroll
@@ -444,6 +452,10 @@ __global__ __launch_bounds__(256) void hier_coef_x6(hier_args a) {
 // positions (16-byte loads and stores, no VALU split); rows past the
 // chunk's end are stored as zeros.  Link, padding rows and outputs as in
 // hier_mfma_f32.
+__host__ __device__ inline int x6_round(int simds, int ncb) {
+  const int n = simds / 4 / ncb / 8 * 8;
+  return n > 8 ? n : 8;
+}
 template <int K>
 __global__ __launch_bounds__(256) void hier_mfma_x6(hier_args a) {
   static_assert(K >= 0 && K <= 31, "K + 1 <= 32 columns");
@@ -463,15 +475,20 @@ __global__ __launch_bounds__(256) void hier_mfma_x6(hier_args a) {
   // chunk group are 8 block ids apart, i.e. on one XCD and dispatched
   // together, so all but the first read the chunk's tiles from that XCD's
   // L2 (launch_hier_x6: a 1-D grid of chunk groups rounded up to 8 x chain
-  // blocks)
+  // blocks).  Chunks from the longest to the shortest, every other round of
+  // x6_round chunk groups (one block per CU) from its end.  Evaluation in us
+  // before and after: J = 1000 of ~400 rows, K = 20, 64 chains 82 -> 77;
+  // K = 8, 256 chains 190 -> 173.
   const int ncb = (a.chains + 31) / 32;
   const int bq = static_cast<int>(blockIdx.x) >> 3;
   const int cbi = bq % ncb;
-  const int64_t ch = (static_cast<int64_t>(bq / ncb) * 8 + (blockIdx.x & 7)) * 4 + w;
-  if (ch >= a.n_chunks) return;  // whole wave; no block barrier follows
-  const int g = a.chunk_group[ch];
-  const int64_t r0 = a.chunk_row0[ch], r1 = a.chunk_row0[ch + 1];
-  const int rows = static_cast<int>(r1 - r0);
+  int64_t cg = static_cast<int64_t>(bq / ncb) * 8 + (blockIdx.x & 7);
+  const int per = x6_round(a.simds, ncb), in = static_cast<int>(cg % per);
+  if ((cg / per) & 1) cg += per - 1 - 2 * in;
+  if (cg * 4 + w >= a.n_chunks) return;  // whole wave; no block barrier follows
+  const hier_chunk hc = a.by_rows[cg * 4 + w];
+  const int64_t ch = hc.id, r0 = hc.row0;
+  const int g = hc.group, rows = hc.rows;
   const int cb = cbi * 32;
   char* const base = lds[w];
   // chain coefficients (w' = log2(e) w, b' = log2(e) b at column K), split
@@ -817,16 +834,19 @@ __global__ __launch_bounds__(1024) void hier_final(hier_args a) {
   put_out<HOST>(out + a.D + 1, bad > 0 ? 1.0 : 0.0);
 }
 
-hipError_t launch_hier_x6(const hier_args& a, dim3 grid, hipStream_t s) {
+hipError_t launch_hier_x6(const hier_args& a, hipStream_t s) {
   // no split copy of X, or no coefficient buffer
-  if ((!a.XS || !a.wsplit) && a.n_chunks > 0) return hipErrorInvalidValue;
+  if ((!a.XS || !a.wsplit || !a.by_rows) && a.n_chunks > 0) return hipErrorInvalidValue;
   const int64_t nc =
       static_cast<int64_t>((a.J + kCoefGroups - 1) / kCoefGroups) * a.chains * 32;
   if (nc > 0)
     hipLaunchKernelGGL(hier_coef_x6, dim3(static_cast<unsigned>((nc + 255) / 256)), dim3(256), 0,
                        s, a);
-  const unsigned ncg8 = static_cast<unsigned>(((a.n_chunks + 3) / 4 + 7) / 8 * 8);
-  grid = dim3(ncg8 * static_cast<unsigned>((a.chains + 31) / 32), 1);
+  const int ncb = (a.chains + 31) / 32;
+  const int64_t ncg = (a.n_chunks + 3) / 4, per = x6_round(a.simds, ncb);
+  // whole rounds: an odd last one is taken from its end
+  const int64_t ncg8 = ncg <= per ? (ncg + 7) / 8 * 8 : (ncg + per - 1) / per * per;
+  const dim3 grid(static_cast<unsigned>(ncg8) * ncb, 1);
   switch (a.K) {
 #define SX_CASE(KK) \
   case KK: hipLaunchKernelGGL((hier_mfma_x6<KK>), grid, dim3(256), 0, s, a); break;
@@ -842,7 +862,14 @@ hipError_t launch_hier_x6(const hier_args& a, dim3 grid, hipStream_t s) {
 }
 
 template <int NH>
-hipError_t launch_hier_mfma(const hier_args& a, dim3 grid, hipStream_t s) {
+hipError_t launch_hier_mfma(const hier_args& a, hipStream_t s) {
+  if (!a.by_rows || a.simds < 4) return hipErrorInvalidValue;
+  const int64_t items = a.n_chunks * ((a.chains + 32 * NH - 1) / (32 * NH));
+  if (items > 0xffffffffll - a.simds) return hipErrorInvalidValue;
+  const unsigned rounds = static_cast<unsigned>((items + a.simds - 1) / a.simds);
+  const unsigned ny = rounds < 32768 ? rounds : 32768;
+  const dim3 grid(rounds > 1 ? a.simds / 4 : static_cast<unsigned>((items + 3) / 4), ny,
+                  (rounds + ny - 1) / ny);
   switch (a.K) {
 #define SX_CASE(KK) \
   case KK: hipLaunchKernelGGL((hier_mfma_f32<KK, NH>), grid, dim3(256), 0, s, a); break;
@@ -894,9 +921,8 @@ hipError_t launch_hier(const hier_args& a, bool fp32, hipStream_t s, bool host_o
         default: return hipErrorInvalidValue;
       }
     } else {
-      const dim3 grid(static_cast<unsigned>((a.n_chunks + 3) / 4), static_cast<unsigned>((a.chains + 31) / 32));
       const hipError_t e =
-          a.x6 && a.K <= 31 ? launch_hier_x6(a, grid, s) : launch_hier_mfma<1>(a, grid, s);
+          a.x6 && a.K <= 31 ? launch_hier_x6(a, s) : launch_hier_mfma<1>(a, s);
       if (e != hipSuccess) return e;
     }
     const hipError_t e = hipGetLastError();

@@ -120,6 +120,11 @@ hipError_t launch_mfma_pass(int family, const double* theta, int64_t D, int C,
 // 128 .. 1024 per data shape); partials per chunk and per group.
 constexpr int kHierChunk = 256;
 constexpr int kHierChunkMin = 128;
+// a chunk as the FP32 batched pass takes it (table sorted by rows)
+struct hier_chunk {
+  int64_t row0;
+  int rows, group, id, pad;
+};
 struct hier_args {
   const double* X;          // N x K row-major (FP64 pass)
   const float* X32;         // N x K row-major (FP32 batched pass)
@@ -133,8 +138,10 @@ struct hier_args {
   const int* chunk_group;   // n_chunks
   const int64_t* chunk_row0;    // n_chunks + 1
   const int64_t* group_chunk0;  // J + 1
+  const hier_chunk* by_rows;    // n_chunks, most rows first
   int64_t n_chunks, theta_stride, out_stride;
   int J, K, D, E, G, chains, propto, jacobian;
+  int simds;  // of the device
   int x6;  // FP32 batches: products on BF16 MFMA in three-term splits (K <= 31)
   double alpha_sd, beta_sd, tau_sd, alpha_const, beta_const, tau_const;
 };
@@ -221,6 +228,7 @@ struct sx_glm {
   uint16_t* d_XS = nullptr;  // split copy of the sign-folded X (FP32, K <= 31)
   int* d_chunk_group = nullptr;
   int64_t *d_chunk_row0 = nullptr, *d_group_chunk0 = nullptr;
+  sx::hier_chunk* d_by_rows = nullptr;
   int64_t n_chunks = 0;
   int hier_chunk = 0;  // rows per chunk at most
   int hier_x6 = 0;     // FP32 batches: products in BF16 three-term splits
