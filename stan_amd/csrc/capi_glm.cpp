@@ -223,24 +223,15 @@ int hier_chunks(sx_glm* m, const int64_t* off, int chunk) {
     }
   }
   gc0.push_back(static_cast<int64_t>(cg.size()));
-  cr0.push_back(m->N);
-  (void)hipFree(m->d_chunk_group);
-  (void)hipFree(m->d_chunk_row0);
   (void)hipFree(m->d_group_chunk0);
   (void)hipFree(m->d_by_rows);
   m->d_by_rows = nullptr;
-  m->d_chunk_group = nullptr;
-  m->d_chunk_row0 = m->d_group_chunk0 = nullptr;
+  m->d_group_chunk0 = nullptr;
   m->n_chunks = static_cast<int64_t>(cg.size());
   m->hier_chunk = chunk;
-  SX_HIP(hipMalloc(&m->d_chunk_group, sizeof(int) * std::max<size_t>(1, cg.size())));
-  SX_HIP(hipMalloc(&m->d_chunk_row0, sizeof(int64_t) * cr0.size()));
   SX_HIP(hipMalloc(&m->d_group_chunk0, sizeof(int64_t) * gc0.size()));
-  if (!cg.empty())
-    SX_HIP(hipMemcpy(m->d_chunk_group, cg.data(), sizeof(int) * cg.size(), hipMemcpyHostToDevice));
-  SX_HIP(hipMemcpy(m->d_chunk_row0, cr0.data(), sizeof(int64_t) * cr0.size(), hipMemcpyHostToDevice));
   SX_HIP(hipMemcpy(m->d_group_chunk0, gc0.data(), sizeof(int64_t) * gc0.size(), hipMemcpyHostToDevice));
-  if (m->precision == SX_FP32 && !cg.empty()) {
+  if (!cg.empty()) {
     // most rows first, by a counting sort over the rows (1 .. chunk)
     std::vector<int64_t> at(static_cast<size_t>(chunk) + 1, 0);
     const auto rows = [&](size_t i) {  // a group's last chunk ends with the group
@@ -656,8 +647,6 @@ void sx_glm_destroy(sx_glm* m) {
   (void)hipFree(m->d_bpart);
   (void)hipFree(m->d_X32);
   (void)hipFree(m->d_XS);
-  (void)hipFree(m->d_chunk_group);
-  (void)hipFree(m->d_chunk_row0);
   (void)hipFree(m->d_group_chunk0);
   (void)hipFree(m->d_by_rows);
   sx::free_workspace(m->hw);
@@ -1116,8 +1105,6 @@ int hier_enqueue(sx_glm* m, hier_workspace& w, const double* d_theta, int C, dou
   a.cpart = w.cpart;
   a.gpart = w.gpart;
   a.wsplit = w.wsplit;
-  a.chunk_group = m->d_chunk_group;
-  a.chunk_row0 = m->d_chunk_row0;
   a.group_chunk0 = m->d_group_chunk0;
   a.by_rows = m->d_by_rows;
   a.simds = m->max_blocks / 2;

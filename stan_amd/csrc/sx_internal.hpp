@@ -120,7 +120,7 @@ hipError_t launch_mfma_pass(int family, const double* theta, int64_t D, int C,
 // 128 .. 1024 per data shape); partials per chunk and per group.
 constexpr int kHierChunk = 256;
 constexpr int kHierChunkMin = 128;
-// a chunk as the FP32 batched pass takes it (table sorted by rows)
+// a chunk as the passes take it (table sorted by rows)
 struct hier_chunk {
   int64_t row0;
   int rows, group, id, pad;
@@ -135,8 +135,6 @@ struct hier_args {
   double* out;              // chains x out_stride: lp, grad[D], status
   double* cpart;            // n_chunks x chains x E
   double* gpart;            // chains x J x G
-  const int* chunk_group;   // n_chunks
-  const int64_t* chunk_row0;    // n_chunks + 1
   const int64_t* group_chunk0;  // J + 1
   const hier_chunk* by_rows;    // n_chunks, most rows first
   int64_t n_chunks, theta_stride, out_stride;
@@ -226,8 +224,7 @@ struct sx_glm {
   // hierarchical model
   float* d_X32 = nullptr;
   uint16_t* d_XS = nullptr;  // split copy of the sign-folded X (FP32, K <= 31)
-  int* d_chunk_group = nullptr;
-  int64_t *d_chunk_row0 = nullptr, *d_group_chunk0 = nullptr;
+  int64_t* d_group_chunk0 = nullptr;
   sx::hier_chunk* d_by_rows = nullptr;
   int64_t n_chunks = 0;
   int hier_chunk = 0;  // rows per chunk at most

@@ -44,3 +44,28 @@ def test_every_chunk_is_taken_once(J, C, kernel):
             lp1, g1 = m.log_prob_grad_batch(th[c:c + 1])
             assert lp1[0] == lp[c] and np.array_equal(g1[0], g[c])
     m.close()
+
+
+# FP64: the same rounds per chain; above 8192 chunks a wave takes several
+@pytest.mark.parametrize("J", [1, 1025, 2048, 2051, 8192, 8193, 9300, 17500])
+def test_every_chunk_is_taken_once_fp64(J):
+    K = 2
+    rng = np.random.default_rng(J)
+    sizes = rng.integers(1, 6, J)
+    sizes[J // 2] = 700  # three chunks
+    off = np.concatenate([[0], np.cumsum(sizes)])
+    X = rng.standard_normal((off[-1], K))
+    y = rng.integers(0, 2, off[-1]).astype(np.int32)
+    prior = (5.0, 2.0, 2.0, 1.0)
+    m = S.GlmModel(S.HIER_LOGIT, X, y, offsets=off, prior=prior, precision=S.FP64)
+    ref = O.GlmData(O.HIER, X, y, offsets=off, prior=prior)
+    th = np.ascontiguousarray(W.random_thetas(m.D, 2, seed=J) * 0.5)
+    lps, gs = m.log_prob_grad_batch(th)
+    for c in range(2):
+        st, lp_r, g_r = ref.lpgrad(th[c], mode=1)
+        assert st == 0
+        lp, g = m.log_prob_grad(th[c])
+        assert lp == lps[c] and np.array_equal(g, gs[c])
+        assert abs(lp - lp_r) <= 1e-12 * max(1.0, abs(lp_r))
+        assert np.linalg.norm(g - g_r) <= 1e-12 * max(1.0, np.linalg.norm(g_r))
+    m.close()
