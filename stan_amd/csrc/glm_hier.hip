@@ -740,105 +740,103 @@ __global__ __launch_bounds__(8 * TW) void hier_groups(hier_args a) {
 
 // Per chain: sums over the group blocks' rows (sixteen fixed interleaved
 // slices of rows, each summed with four accumulators, then combined in
-// order), priors, Jacobian, output.  Every load of a slice is independent
-// and sixteen are issued before they are added, so the sums are bandwidth-
-// rather than latency-bound.
+// order), priors, Jacobian, output.  One block per chain, so latency-bound:
+// every load of a slice is independent and sixteen are issued before they
+// are added; the prior terms are computed before the sums are needed; and
+// the last thread reads the terms it adds in order eight at a time.  us at
+// J = 1000, K = 20, with the rows loaded four at a time, the priors after
+// the sums and one term read per add, and this: 1 chain 6.4 / 4.6, 64 chains
+// 6.8 / 4.8.
 template <bool HOST>
 __global__ __launch_bounds__(1024) void hier_final(hier_args a) {
   __shared__ double red[16][64];
   __shared__ double st[128];
+  // log-density terms in the order they are added (alpha, beta_k, then per
+  // tau_k the prior and the Jacobian term), zeros past them
+  __shared__ double seq[104];
   const int c = blockIdx.x;
   const int K = a.K;
   const double* th = a.theta + static_cast<int64_t>(c) * a.theta_stride;
   double* out = a.out + static_cast<int64_t>(c) * a.out_stride;
-  const int sl = threadIdx.x >> 6;
+  const int sl = threadIdx.x >> 6, ln = threadIdx.x & 63;
   const int R = (a.J + kGroupsPerBlock - 1) / kGroupsPerBlock;  // rows per chain
+  // prior and Jacobian terms in parallel: wave 0 lane 0 alpha, lanes 1..K
+  // beta; wave 1 lanes 0..K tau; gp: the prior's share of the gradient (tau:
+  // minus its square)
+  const int nseq = 3 * K + 3;
+  double gp = 0.0;
+  const bool own = sl < 2 && ln <= K;
+  if (own) {
+    if (sl == 0) {
+      const double sd = ln == 0 ? a.alpha_sd : a.beta_sd;
+      double t = 0.0;
+      if (sd > 0) {
+        const double zz = th[ln] / sd;
+        t = -0.5 * zz * zz + (a.propto ? 0.0 : (ln == 0 ? a.alpha_const : a.beta_const));
+        gp = -th[ln] / (sd * sd);
+      }
+      seq[ln] = t;
+    } else {
+      const double v = th[1 + K + ln];
+      const double tau = exp(v);
+      double t = 0.0;
+      if (a.tau_sd > 0) {
+        const double zz = tau / a.tau_sd;
+        t = -0.5 * zz * zz + (a.propto ? 0.0 : a.tau_const);
+        gp = zz;
+      }
+      seq[K + 1 + 2 * ln] = t;
+      seq[K + 2 + 2 * ln] = a.jacobian ? v : 0.0;
+    }
+  } else if (sl == 2 && nseq + ln < 104) {
+    seq[nseq + ln] = 0.0;
+  }
+  if (sl == 2 && nseq + ln + 64 < 104) seq[nseq + ln + 64] = 0.0;
   for (int e0 = 0; e0 < a.G; e0 += 64) {
-    const int e = e0 + (threadIdx.x & 63);
+    const int e = e0 + ln;
     if (e < a.G) {
-      const double* gp = a.gpart + static_cast<int64_t>(c) * R * a.G + e;
+      const double* gq = a.gpart + static_cast<int64_t>(c) * R * a.G + e;
       double v[4] = {0.0, 0.0, 0.0, 0.0};
-      int g = sl;
-      // sixteen loads in flight, added in the order of the 4-load steps
-      for (; g + 240 < R; g += 256) {
+      for (int g = sl; g < R; g += 256) {
         double x[16];
 #pragma unroll
-        for (int u = 0; u < 16; ++u) x[u] = gp[static_cast<int64_t>(g + 16 * u) * a.G];
+        for (int u = 0; u < 16; ++u) x[u] = g + 16 * u < R ? gq[static_cast<int64_t>(g + 16 * u) * a.G] : 0.0;
 #pragma unroll
-        for (int u = 0; u < 16; ++u) v[u & 3] += x[u];
+        for (int u = 0; u < 16; ++u)
+          if (g + 16 * u < R) v[u & 3] += x[u];
       }
-      for (; g + 48 < R; g += 64) {
-#pragma unroll
-        for (int u = 0; u < 4; ++u) v[u] += gp[static_cast<int64_t>(g + 16 * u) * a.G];
-      }
-      for (int u = 0; g < R; g += 16, ++u) v[u] += gp[static_cast<int64_t>(g) * a.G];
-      red[sl][threadIdx.x & 63] = (v[0] + v[1]) + (v[2] + v[3]);
+      red[sl][ln] = (v[0] + v[1]) + (v[2] + v[3]);
     }
     __syncthreads();
-    if (threadIdx.x < 64 && e0 + static_cast<int>(threadIdx.x) < a.G) {
-      double t = 0.0;
+    if (sl == 0 && e < a.G) {
+      double x[16], t = 0.0;
 #pragma unroll
-      for (int i = 0; i < 16; ++i) t += red[i][threadIdx.x];
-      st[e0 + threadIdx.x] = t;
+      for (int i = 0; i < 16; ++i) x[i] = red[i][ln];
+#pragma unroll
+      for (int i = 0; i < 16; ++i) t += x[i];
+      st[e] = t;
     }
     __syncthreads();
   }
-  // prior and Jacobian terms in parallel: wave 0 lane 0 alpha, lanes
-  // 1..K beta; wave 1 lanes 0..K tau.  Thread 0 then adds the log-density
-  // terms in a fixed order (alpha, beta_k, then per tau_k the prior and the
-  // Jacobian term).
-  __shared__ double lpa[33], lpt[2][33];
-  const int ln = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  if (wv == 0 && ln <= K) {
-    if (ln == 0) {
-      double ga = st[0], t = 0.0;
-      if (a.alpha_sd > 0) {
-        const double zz = th[0] / a.alpha_sd;
-        t = -0.5 * zz * zz + (a.propto ? 0.0 : a.alpha_const);
-        ga += -th[0] / (a.alpha_sd * a.alpha_sd);
-      }
-      put_out<HOST>(out + 1, ga);
-      lpa[0] = t;
+  if (own) {
+    double gv = st[sl == 0 ? ln : K + 1 + ln];
+    if (sl == 0) {
+      if ((ln == 0 ? a.alpha_sd : a.beta_sd) > 0) gv += gp;
     } else {
-      const int k = ln - 1;
-      double gb = st[1 + k], t = 0.0;
-      const double bk = th[1 + k];
-      if (a.beta_sd > 0) {
-        const double zz = bk / a.beta_sd;
-        t = -0.5 * zz * zz + (a.propto ? 0.0 : a.beta_const);
-        gb += -bk / (a.beta_sd * a.beta_sd);
-      }
-      put_out<HOST>(out + 2 + k, gb);
-      lpa[ln] = t;
+      if (a.tau_sd > 0) gv = fma(-gp, gp, gv);
+      if (a.jacobian) gv += 1.0;
     }
-  } else if (wv == 1 && ln <= K) {
-    const int k = ln;
-    const double v = th[1 + K + k];
-    const double tau = exp(v);
-    double gv = st[K + 1 + k], t = 0.0, jt = 0.0;
-    if (a.tau_sd > 0) {
-      const double zz = tau / a.tau_sd;
-      t = -0.5 * zz * zz + (a.propto ? 0.0 : a.tau_const);
-      gv += -zz * zz;
-    }
-    if (a.jacobian) {
-      jt = v;
-      gv += 1.0;
-    }
-    put_out<HOST>(out + 2 + K + k, gv);
-    lpt[0][k] = t;
-    lpt[1][k] = jt;
+    put_out<HOST>(out + 1 + (sl == 0 ? ln : K + 1 + ln), gv);
   }
-  __syncthreads();
   if (threadIdx.x != 0) return;
   double lp = st[2 * K + 2];
   double bad = st[2 * K + 3];
-  if (a.alpha_sd > 0) lp += lpa[0];
-  if (a.beta_sd > 0)
-    for (int k = 0; k < K; ++k) lp += lpa[1 + k];
-  for (int k = 0; k <= K; ++k) {
-    if (a.tau_sd > 0) lp += lpt[0][k];
-    if (a.jacobian) lp += lpt[1][k];
+  for (int i = 0; i < nseq; i += 8) {
+    double x[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) x[u] = seq[i + u];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) lp += x[u];
   }
   lp += -0.5 * st[2 * K + 4];
   if (!a.propto) lp += -static_cast<double>(a.J) * (K + 1) * kHalfLog2PiH;
