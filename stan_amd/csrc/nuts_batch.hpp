@@ -83,8 +83,8 @@ struct batch_args {
   // failure injection for tests: waits expect a tag no part writes, so
   // every exchange times out after spin_limit polls
   int xnever;
-  // phase turns a chain may take per launch before it yields (large D:
-  // the vector work of a deep subtree's merges would set the step time)
+  // phase turns a chain may take per launch before it yields (else the
+  // vector work of a deep subtree's merges would set the step time)
   int phase_budget;
 };
 
