@@ -545,7 +545,9 @@ int sx_glm_create_ex(sx_glm** out, int family, const double* X, const void* y, i
   if (hipMalloc(&m->d_theta, sizeof(double) * (m->D + 1)) != hipSuccess) return fail(SX_ENOMEM);
   if (hipMalloc(&m->d_out, sizeof(double) * (m->D + 2)) != hipSuccess) return fail(SX_ENOMEM);
   if (hipHostMalloc(&m->h_theta, sizeof(double) * (m->D + 1)) != hipSuccess) return fail(SX_ENOMEM);
-  if (hipHostMalloc(&m->h_out, sizeof(double) * (m->D + 2)) != hipSuccess) return fail(SX_ENOMEM);
+  // the kernels' stores reach it while they run, whatever the process's default
+  if (hipHostMalloc(&m->h_out, sizeof(double) * (m->D + 2), hipHostMallocCoherent) != hipSuccess)
+    return fail(SX_ENOMEM);
   if (hipEventCreate(&m->ev0) != hipSuccess || hipEventCreate(&m->ev1) != hipSuccess)
     return fail(SX_EDEVICE);
   const int max_blocks = 8 * cus;
@@ -701,21 +703,33 @@ void unset_words(double* w, size_t n) {
 }
 
 // Waits until the kernels on m's stream have stored n output words (each
-// one aligned 8-byte store, so a word that is no longer kUnset is whole).
+// one aligned 8-byte store, so a word that is no longer kUnset is whole) and
+// copies them to dst (unless NULL) as they arrive.
+// Every word that is read must be among them: a word says nothing about
+// another one, also not of an earlier launch, whose stores only the stream's
+// completion publishes to the host.
 // Watching the words returns a few microseconds before the stream's
-// completion signal would (4 of 20 us for a small evaluation); after 5 ms
-// the stream is waited for instead, which also reports a failed launch.
-int wait_words(sx_glm* m, const double* w, size_t n) {
-  const auto start = std::chrono::steady_clock::now();
+// completion signal would (4 of 20 us for a small evaluation); 5 ms after
+// `start` the stream is waited for instead, which also reports a failed
+// launch.
+int take_words(sx_glm* m, const double* w, size_t n, double* dst,
+               std::chrono::steady_clock::time_point start) {
   bool synced = false;
   unsigned spins = 0;
+  const auto unset = [w](size_t i) {
+    return __atomic_load_n(reinterpret_cast<const uint64_t*>(w + i), __ATOMIC_ACQUIRE) == kUnset;
+  };
   for (size_t i = 0; i < n;) {
-    if (__atomic_load_n(reinterpret_cast<const uint64_t*>(w + i), __ATOMIC_ACQUIRE) != kUnset) {
-      ++i;
+    const size_t e = std::min(n, i + 64);
+    bool any = false;
+    for (size_t k = i; k < e; ++k) any |= unset(k);
+    if (!any) {
+      if (dst) std::memcpy(dst + i, w + i, (e - i) * sizeof(double));
+      i = e;
     } else if (synced) {
       set_error("log_prob: the device stored no result");
       return SX_EDEVICE;
-    } else if (++spins % 1024 == 0 &&
+    } else if (++spins % 256 == 0 &&
                std::chrono::steady_clock::now() - start > std::chrono::milliseconds(5)) {
       SX_HIP(hipStreamSynchronize(m->stream));
       synced = true;
@@ -763,25 +777,27 @@ int eval(sx_glm* m, const double* theta, int propto, int jacobian, double* lp,
   std::memcpy(m->h_theta, theta, D * sizeof(double));
   int rc;
   if (m->family == SX_HIER_LOGIT) {
-    // the last launch (hier_final) starts after the z gradients of the one
-    // before are stored: watch what it stores
-    const size_t head = 2 * static_cast<size_t>(m->K) + 3;
-    unset_words(m->h_out, head);
-    unset_words(m->h_out + D + 1, 1);
+    // the words are reset while theta is on its way
     SX_HIP(hipMemcpyAsync(m->d_theta, m->h_theta, D * sizeof(double), hipMemcpyHostToDevice,
                           m->stream));
+    unset_words(m->h_out, D + 2);
     rc = sx::hier_enqueue(m, m->hw, m->d_theta, 1, m->h_out, propto, jacobian, false, m->stream,
                           true);
-    if (rc == SX_OK) rc = wait_words(m, m->h_out, head);
-    if (rc == SX_OK) rc = wait_words(m, m->h_out + D + 1, 1);
   } else {
     unset_words(m->h_out, D + 2);
     rc = sx::plain_eval(m, propto, jacobian);
-    if (rc == SX_OK) rc = wait_words(m, m->h_out, D + 2);
   }
   if (rc) return rc;
-  *lp = m->h_out[0];
-  if (grad) std::memcpy(grad, m->h_out + 1, D * sizeof(double));
+  // the words in the order in which they are stored: the hierarchical
+  // model's z gradients come a launch before the others
+  const auto start = std::chrono::steady_clock::now();
+  const size_t head = m->family == SX_HIER_LOGIT ? 2 * static_cast<size_t>(m->K) + 3 : D + 1;
+  rc = take_words(m, m->h_out + head, D + 1 - head, grad ? grad + head - 1 : nullptr, start);
+  if (rc == SX_OK)
+    rc = take_words(m, m->h_out + 1, head - 1, grad, start);
+  if (rc == SX_OK) rc = take_words(m, m->h_out, 1, lp, start);
+  if (rc == SX_OK) rc = take_words(m, m->h_out + D + 1, 1, nullptr, start);
+  if (rc) return rc;
   if (m->h_out[D + 1] != 0.0) {
     set_error(domain_message(m->family));
     return SX_EDOMAIN;

@@ -1,0 +1,329 @@
+// Host check of the evaluation calls (stan_amd/csrc/capi_glm.cpp) against a
+// stand-in HIP runtime: device memory is host memory, a stream is a thread
+// that works its queue off, and the kernels are replaced by a function of
+// theta that is as simple as it is different from point to point.  The
+// stand-in shows what the hardware shows rarely or never: stores that reach
+// the host in another order than they were issued, work that is still queued
+// when a call returns, and allocations that fail.
+//   glm_calls_check <scenario>   prints "ok" or what went wrong
+#include <malloc.h>
+
+#include <chrono>
+#include <condition_variable>
+#include <cstdio>
+#include <deque>
+#include <functional>
+#include <map>
+
+#include "../../stan_amd/csrc/capi_glm.cpp"
+
+namespace {
+
+// ---- the stand-in runtime -------------------------------------------------
+
+struct stream_queue {
+  std::mutex mu;
+  std::condition_variable cv;
+  std::deque<std::function<void()>> q;
+  size_t pending = 0;
+  bool stop = false;
+  std::thread th;
+  stream_queue() : th([this] { work(); }) {}
+  ~stream_queue() {
+    {
+      std::lock_guard<std::mutex> l(mu);
+      stop = true;
+    }
+    cv.notify_all();
+    th.join();
+  }
+  void work();
+  void push(std::function<void()> f) {
+    std::lock_guard<std::mutex> l(mu);
+    q.push_back(std::move(f));
+    ++pending;
+    cv.notify_all();
+  }
+  void wait() {
+    std::unique_lock<std::mutex> l(mu);
+    cv.wait(l, [this] { return pending == 0; });
+  }
+};
+
+int g_delay_us = 0;          // before every queued operation
+bool g_fail_launch = false;  // kernel launches are refused
+bool g_no_store = false;     // kernels run and store nothing
+bool g_fail_pinned = false;  // no pinned memory
+size_t g_limit = SIZE_MAX, g_used = 0;  // device memory
+std::map<void*, size_t> g_dev;
+int g_pinned_calls = 0;
+
+void pause_us(int us) {
+  if (us > 0) std::this_thread::sleep_for(std::chrono::microseconds(us));
+}
+
+void stream_queue::work() {
+  std::unique_lock<std::mutex> l(mu);
+  while (true) {
+    cv.wait(l, [this] { return stop || !q.empty(); });
+    if (q.empty()) return;
+    std::function<void()> f = std::move(q.front());
+    q.pop_front();
+    l.unlock();
+    pause_us(g_delay_us);
+    f();
+    l.lock();
+    --pending;
+    cv.notify_all();
+  }
+}
+
+stream_queue* queue_of(hipStream_t s) { return reinterpret_cast<stream_queue*>(s); }
+
+// the stand-in density: distinct for every theta and parameter
+double value(const double* th, int D) {
+  double s = 0;
+  for (int i = 0; i < D; ++i) s += (i + 1) * th[i];
+  return s;
+}
+double slope(const double* th, int i) { return 2.0 * th[i] + i; }
+
+void store(double* out, size_t i, double v) {
+  __atomic_store_n(reinterpret_cast<uint64_t*>(out + i), *reinterpret_cast<uint64_t*>(&v),
+                   __ATOMIC_RELAXED);
+}
+
+// one chain's outputs; the words of `late` reach the host after the others
+void put(const double* th, double* out, int D, size_t late0, size_t late1) {
+  if (g_no_store) return;
+  const auto one = [&](size_t i) {
+    store(out, i, i == 0 ? value(th, D) : i == static_cast<size_t>(D) + 1 ? 0.0 : slope(th, i - 1));
+  };
+  for (size_t i = D + 2; i-- > 0;)
+    if (i < late0 || i >= late1) one(i);
+  if (late0 < late1) pause_us(3000);
+  for (size_t i = late0; i < late1; ++i) one(i);
+}
+
+}  // namespace
+
+extern "C" {
+
+hipError_t hipGetDevice(int* d) { return *d = 0, hipSuccess; }
+hipError_t hipSetDevice(int) { return hipSuccess; }
+hipError_t hipGetDeviceCount(int* n) { return *n = 1, hipSuccess; }
+hipError_t hipGetDevicePropertiesR0600(hipDeviceProp_tR0600* p, int) {
+  std::memset(static_cast<void*>(p), 0, sizeof *p);
+  p->multiProcessorCount = 256;
+  return hipSuccess;
+}
+const char* hipGetErrorString(hipError_t) { return "stand-in error"; }
+hipError_t hipMalloc(void** p, size_t n) {
+  *p = nullptr;
+  if (n > g_limit - std::min(g_limit, g_used)) return hipErrorOutOfMemory;
+  *p = std::calloc(1, std::max<size_t>(n, 1));
+  g_dev[*p] = n;
+  g_used += n;
+  return hipSuccess;
+}
+hipError_t hipFree(void* p) {
+  if (!p) return hipSuccess;
+  g_used -= g_dev[p];
+  g_dev.erase(p);
+  std::free(p);
+  return hipSuccess;
+}
+hipError_t hipHostMalloc(void** p, size_t n, unsigned) {
+  *p = nullptr;
+  if (g_fail_pinned) return hipErrorOutOfMemory;
+  ++g_pinned_calls;
+  *p = std::calloc(1, n);
+  return hipSuccess;
+}
+hipError_t hipHostFree(void* p) { return std::free(p), hipSuccess; }
+hipError_t hipMemcpy(void* d, const void* s, size_t n, hipMemcpyKind) {
+  return std::memcpy(d, s, n), hipSuccess;
+}
+hipError_t hipMemset(void* d, int v, size_t n) { return std::memset(d, v, n), hipSuccess; }
+hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind, hipStream_t st) {
+  queue_of(st)->push([=] { std::memcpy(d, s, n); });
+  return hipSuccess;
+}
+hipError_t hipMemsetAsync(void* d, int v, size_t n, hipStream_t st) {
+  queue_of(st)->push([=] { std::memset(d, v, n); });
+  return hipSuccess;
+}
+hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) {
+  return *s = reinterpret_cast<hipStream_t>(new stream_queue), hipSuccess;
+}
+hipError_t hipStreamSynchronize(hipStream_t s) { return queue_of(s)->wait(), hipSuccess; }
+hipError_t hipStreamDestroy(hipStream_t s) { return delete queue_of(s), hipSuccess; }
+hipError_t hipEventCreate(hipEvent_t* e) { return *e = nullptr, hipSuccess; }
+hipError_t hipEventDestroy(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
+hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventElapsedTime(float* ms, hipEvent_t, hipEvent_t) { return *ms = 1.f, hipSuccess; }
+
+}  // extern "C"
+
+namespace sx {
+
+int noalloc_setup(int) { return SX_OK; }
+
+tile_geom make_geom(int64_t N, int64_t K, int L, int smax) {
+  tile_geom g;
+  g.L = L;
+  for (g.lgL = 0; (1 << g.lgL) < L;) ++g.lgL;
+  g.R = 64 / L;
+  g.S = static_cast<int>((K + L - 1) / L);
+  g.smax = smax;
+  g.T = (N + g.R - 1) / g.R;
+  return g;
+}
+hipError_t launch_tile_x_f64(const double*, double*, int64_t, int64_t, const tile_geom&,
+                             hipStream_t) {
+  return hipSuccess;
+}
+hipError_t launch_split_x(const double*, uint16_t*, uint16_t*, int64_t, int64_t, int64_t, int64_t,
+                          hipStream_t) {
+  return hipSuccess;
+}
+hipError_t launch_prep_y(const void*, float*, int, int64_t, int64_t, hipStream_t) {
+  return hipSuccess;
+}
+// points and results of a batch, one chain after the other
+static hipError_t batch(const double* theta, int64_t ts, double* out, int64_t os, int D, int C,
+                        double* scratch, int64_t per_chain, hipStream_t s, size_t late0 = 0,
+                        size_t late1 = 0) {
+  if (g_fail_launch) return hipErrorInvalidValue;
+  queue_of(s)->push([=] {
+    for (int c = 0; c < C; ++c) {
+      for (int64_t i = 0; i < per_chain; ++i) scratch[c * per_chain + i] = c;
+      put(theta + c * ts, out + c * os, D, late0, late1);
+    }
+  });
+  return hipSuccess;
+}
+hipError_t launch_pass_f64(int, const tile_geom&, const pass_args& a, int blocks, int,
+                           hipStream_t s, bool) {
+  return batch(a.theta, a.theta_stride, a.out, a.out_stride, a.D, a.chains, a.partials,
+               static_cast<int64_t>(a.E) * blocks, s);
+}
+hipError_t launch_eval_f64(int, const tile_geom&, const pass_args& a, const double* h_theta, int,
+                           int, hipStream_t s) {
+  if (g_fail_launch) return hipErrorInvalidValue;
+  const std::vector<double> th(h_theta, h_theta + a.D);  // carried by the launch
+  double* out = a.out;
+  queue_of(s)->push([=] { put(th.data(), out, static_cast<int>(th.size()), 2, 4); });
+  return hipSuccess;
+}
+hipError_t launch_mfma_pass(int, const double* theta, int64_t D, int C, const mx_args&,
+                            const pass_args& pa, hipStream_t s) {
+  return batch(theta, D, pa.out, pa.out_stride, static_cast<int>(D), C, nullptr, 0, s);
+}
+// To the host, the z gradients of the launch before the last are the last to
+// arrive: nothing between the two launches publishes them to it.
+hipError_t launch_hier(const hier_args& a, bool, hipStream_t s, bool host_out) {
+  const size_t z0 = 2 * static_cast<size_t>(a.K) + 3, z1 = static_cast<size_t>(a.D) + 1;
+  return batch(a.theta, a.theta_stride, a.out, a.out_stride, a.D, a.chains, a.cpart, a.E, s,
+               host_out ? z0 : 0, host_out ? z1 : 0);
+}
+
+}  // namespace sx
+
+// ---- scenarios -------------------------------------------------------------
+
+namespace {
+
+int g_bad = 0;
+#define CHECK(cond)                                                  \
+  do {                                                               \
+    if (!(cond) && ++g_bad < 10)                                     \
+      std::printf("line %d: %s (%s)\n", __LINE__, #cond, sx_last_error()); \
+  } while (0)
+
+sx_glm* make(int family, int64_t N, int64_t K, int64_t J, int precision) {
+  std::vector<double> X(N * K, 0.5), yd(N, 1.0);
+  std::vector<int32_t> yi(N, 1);
+  std::vector<int64_t> off(J + 1);
+  for (int64_t j = 0; j <= J; ++j) off[j] = N * j / std::max<int64_t>(J, 1);
+  sx_glm* m = nullptr;
+  const void* y = family == SX_NORMAL ? static_cast<const void*>(yd.data()) : yi.data();
+  CHECK(sx_glm_create(&m, family, X.data(), y, N, K, J ? off.data() : nullptr, J, precision,
+                      nullptr, 0) == SX_OK);
+  return m;
+}
+
+std::vector<double> points(int64_t C, int64_t D, int seed) {
+  std::vector<double> th(C * D);
+  for (size_t i = 0; i < th.size(); ++i) th[i] = 0.25 * seed + 0.001 * (i % 977) + 1e-6 * i;
+  return th;
+}
+
+void check_chain(const double* th, int D, double lp, const double* g) {
+  CHECK(lp == value(th, D));
+  for (int i = 0; i < D; ++i) CHECK(g[i] == slope(th, i));
+}
+
+void check_batch(sx_glm* m, int64_t C, int seed, int64_t from = 0) {
+  const std::vector<double> th = points(C, m->D, seed);
+  std::vector<double> lp(C), g(C * m->D);
+  CHECK(sx_glm_logp_grad_batch(m, th.data(), C, 1, 1, lp.data(), g.data()) == SX_OK);
+  for (int64_t c = from; c < C; ++c)
+    check_chain(th.data() + c * m->D, static_cast<int>(m->D), lp[c], g.data() + c * m->D);
+}
+
+void check_single(sx_glm* m, int seed) {
+  const std::vector<double> th = points(1, m->D, seed);
+  double lp = 0;
+  std::vector<double> g(m->D);
+  CHECK(sx_glm_logp_grad(m, th.data(), 1, 1, &lp, g.data()) == SX_OK);
+  check_chain(th.data(), static_cast<int>(m->D), lp, g.data());
+}
+
+// Single evaluations return this call's results, whatever the order in which
+// the words reach the host.
+void single_fresh() {
+  sx_glm* h = make(SX_HIER_LOGIT, 400, 3, 50, SX_FP64);
+  sx_glm* m = make(SX_NORMAL, 300, 7, 0, SX_FP64);
+  for (int i = 1; i <= 4; ++i) {
+    check_single(h, i);
+    check_single(m, i);
+  }
+  sx_glm_destroy(h);
+  sx_glm_destroy(m);
+}
+
+// A device that takes longer than the host watches its words for.
+void single_slow() {
+  sx_glm* h = make(SX_HIER_LOGIT, 60, 2, 5, SX_FP64);
+  sx_glm* m = make(SX_LOGIT, 60, 3, 0, SX_FP64);
+  g_delay_us = 20000;
+  for (int i = 1; i <= 2; ++i) {
+    check_single(h, i);
+    check_single(m, i);
+  }
+  // a launch that stores nothing is an error, not the last call's result
+  g_no_store = true;
+  double lp = 0;
+  std::vector<double> g(h->D), th = points(1, h->D, 3);
+  CHECK(sx_glm_logp_grad(h, th.data(), 1, 1, &lp, g.data()) == SX_EDEVICE);
+  CHECK(sx_glm_logp_grad(m, th.data(), 1, 1, &lp, g.data()) == SX_EDEVICE);
+  g_no_store = false;
+  g_delay_us = 0;
+  check_single(h, 4);
+  check_single(m, 4);
+  sx_glm_destroy(h);
+  sx_glm_destroy(m);
+}
+
+}  // namespace
+
+int main(int argc, char** argv) {
+  const std::string what = argc > 1 ? argv[1] : "";
+  if (what == "single_fresh") single_fresh();
+  else if (what == "single_slow") single_slow();
+  else return std::printf("unknown scenario\n"), 2;
+  if (!g_bad) std::printf("ok\n");
+  return g_bad != 0;
+}

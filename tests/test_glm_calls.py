@@ -1,0 +1,33 @@
+"""The evaluation calls' host side on a stand-in HIP runtime (no GPU): what
+they return when stores reach the host late and out of order, what they leave
+queued, and what they do when memory is refused (tests/cpp/glm_calls_check.cpp
+says how)."""
+import os
+import subprocess
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
+
+
+@pytest.fixture(scope="module")
+def check(tmp_path_factory):
+    exe = str(tmp_path_factory.mktemp("cpp") / "glm_calls_check")
+    subprocess.run(["g++", "-O1", "-std=c++17", "-pthread", "-D__HIP_PLATFORM_AMD__",
+                    "-I" + os.path.join(ROCM, "include"), "-o", exe,
+                    os.path.join(HERE, "cpp", "glm_calls_check.cpp")], check=True)
+
+    def run(scenario):
+        out = subprocess.run([exe, scenario], capture_output=True, text=True, timeout=100)
+        assert out.returncode == 0 and out.stdout.strip() == "ok", out.stdout + out.stderr
+
+    return run
+
+
+@pytest.mark.parametrize("scenario", ["single_fresh", "single_slow"])
+def test_single_evaluations(check, scenario):
+    """Every value is this call's own: also those that arrive after the log
+    density and the status, and those of a launch that takes longer than the
+    host watches the output; a launch that stores nothing is an error."""
+    check(scenario)
