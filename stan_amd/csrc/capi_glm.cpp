@@ -740,6 +740,16 @@ int take_words(sx_glm* m, const double* w, size_t n, double* dst,
   return SX_OK;
 }
 
+// A call that returns with an error leaves nothing queued: its copies read
+// the caller's points, or buffers that the next call fills while it runs.
+struct drain_on_error {
+  sx_glm* m;
+  bool done = false;
+  ~drain_on_error() {
+    if (!done) (void)hipStreamSynchronize(m->stream);
+  }
+};
+
 const char* domain_message(int family) {
   return family == SX_LOGIT ? "bernoulli_logit_glm_lpmf: linear predictor or log density is not finite"
          : family == SX_NORMAL
@@ -775,6 +785,7 @@ int eval(sx_glm* m, const double* theta, int propto, int jacobian, double* lp,
     return SX_EDOMAIN;
   }
   std::memcpy(m->h_theta, theta, D * sizeof(double));
+  drain_on_error queued{m};
   int rc;
   if (m->family == SX_HIER_LOGIT) {
     // the words are reset while theta is on its way
@@ -798,6 +809,7 @@ int eval(sx_glm* m, const double* theta, int propto, int jacobian, double* lp,
   if (rc == SX_OK) rc = take_words(m, m->h_out, 1, lp, start);
   if (rc == SX_OK) rc = take_words(m, m->h_out + D + 1, 1, nullptr, start);
   if (rc) return rc;
+  queued.done = true;
   if (m->h_out[D + 1] != 0.0) {
     set_error(domain_message(m->family));
     return SX_EDOMAIN;
@@ -1232,6 +1244,7 @@ int batch_call(sx_glm* m, const double* theta, int64_t C, int64_t slab, bool che
   if (!pinned && m->bout.size() < most / sizeof(double)) m->bout.resize(most / sizeof(double));
   const double* const out = pinned ? m->h_batch : m->bout.data();
   int worst = SX_OK;
+  drain_on_error queued{m};
   for (int64_t b = 0; b < C; b += slab) {
     const int64_t n = std::min(slab, C - b);
     const double* th = theta + b * D;
@@ -1264,6 +1277,7 @@ int batch_call(sx_glm* m, const double* theta, int64_t C, int64_t slab, bool che
           std::memcpy(grad + (b + c) * D, out + c * (D + 2) + 1, row);
       });
   }
+  queued.done = true;
   return worst;
 }
 

@@ -317,12 +317,46 @@ void single_slow() {
   sx_glm_destroy(m);
 }
 
+// A call that fails leaves nothing queued: its points may be freed, its
+// buffers used again.
+void failed_calls_drain() {
+  g_delay_us = 5000;
+  for (int prec : {SX_FP64, SX_FP32}) {
+    sx_glm* h = make(SX_HIER_LOGIT, 90, 3, 30, prec);
+    for (int64_t C : {1, 3, 100, 2000}) {  // below, between and above the pinned buffer's limits
+      std::vector<double> th = points(C, h->D, 1), lp(C), g(C * h->D);
+      g_fail_launch = true;
+      CHECK(sx_glm_logp_grad_batch(h, th.data(), C, 1, 1, lp.data(), g.data()) == SX_EDEVICE);
+      CHECK(queue_of(h->stream)->pending == 0);
+      if (C == 1) {
+        CHECK(sx_glm_logp_grad(h, th.data(), 1, 1, lp.data(), g.data()) == SX_EDEVICE);
+        CHECK(queue_of(h->stream)->pending == 0);
+      }
+      g_fail_launch = false;
+      check_batch(h, C, 2);
+    }
+    check_single(h, 3);
+    sx_glm_destroy(h);
+  }
+  sx_glm* m = make(SX_LOGIT, 64, 4, 0, SX_FP64);
+  for (int64_t C : {1, 2, 3000}) {
+    std::vector<double> th = points(C, m->D, 1), lp(C), g(C * m->D);
+    g_fail_launch = true;
+    CHECK(sx_glm_logp_grad_batch(m, th.data(), C, 1, 1, lp.data(), g.data()) == SX_EDEVICE);
+    CHECK(queue_of(m->stream)->pending == 0);
+    g_fail_launch = false;
+    check_batch(m, C, 2);
+  }
+  sx_glm_destroy(m);
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
   const std::string what = argc > 1 ? argv[1] : "";
   if (what == "single_fresh") single_fresh();
   else if (what == "single_slow") single_slow();
+  else if (what == "failed_calls_drain") failed_calls_drain();
   else return std::printf("unknown scenario\n"), 2;
   if (!g_bad) std::printf("ok\n");
   return g_bad != 0;

@@ -31,3 +31,9 @@ def test_single_evaluations(check, scenario):
     density and the status, and those of a launch that takes longer than the
     host watches the output; a launch that stores nothing is an error."""
     check(scenario)
+
+
+def test_failed_calls_leave_nothing_queued(check):
+    """A call whose launch is refused waits for the copies it has queued: they
+    read the caller's points or buffers that the next call fills."""
+    check("failed_calls_drain")
