@@ -1237,10 +1237,13 @@ int batch_call(sx_glm* m, const double* theta, int64_t C, int64_t slab, bool che
   slab = std::max<int64_t>(
       1, std::min<int64_t>({C, slab, static_cast<int64_t>(kPinnedBytes / (row + 16))}));
   const size_t most = slab * (row + 16);
-  const bool pinned = most < kSmallBytes || most >= kLargeBytes;
   int rc = ensure_batch_staging(m, slab);
-  if (rc == SX_OK && pinned) rc = ensure_batch_pinned(m, slab);
   if (rc) return rc;
+  bool pinned = most < kSmallBytes || most >= kLargeBytes;
+  if (pinned && ensure_batch_pinned(m, slab) != SX_OK) {  // refused: pageable
+    (void)hipGetLastError();
+    pinned = false;
+  }
   if (!pinned && m->bout.size() < most / sizeof(double)) m->bout.resize(most / sizeof(double));
   const double* const out = pinned ? m->h_batch : m->bout.data();
   int worst = SX_OK;
@@ -1286,18 +1289,47 @@ int batch_call(sx_glm* m, const double* theta, int64_t C, int64_t slab, bool che
 // bitwise its single evaluation's.
 constexpr size_t kSlabBytes = size_t(256) << 20;
 
+int ensure_batch_partials(sx_glm* m, int64_t C) {
+  if (m->bpart_cap >= C) return SX_OK;
+  (void)hipFree(m->d_bpart);
+  m->d_bpart = nullptr;
+  m->bpart_cap = 0;
+  SX_HIP(hipMalloc(&m->d_bpart, sizeof(double) * (m->K + 3) * m->blocks * C));
+  m->bpart_cap = C;
+  return SX_OK;
+}
+
+// One chain after the other, in the context's own buffers.
+int one_by_one(sx_glm* m, const double* theta, int64_t C, int propto, int jacobian, double* lp,
+               double* grad) {
+  int worst = SX_OK;
+  for (int64_t c = 0; c < C; ++c) {
+    const int rc = eval(m, theta + c * m->D, propto, jacobian, lp + c,
+                        grad ? grad + c * m->D : nullptr);
+    if (rc == SX_EDOMAIN) {
+      lp[c] = -INFINITY;
+      worst = SX_EDOMAIN;
+    } else if (rc) {
+      return rc;
+    }
+  }
+  return worst;
+}
+
 int fp64_batch(sx_glm* m, const double* theta, int64_t C, int propto, int jacobian, double* lp,
                double* grad) {
   SX_HIP(hipSetDevice(m->device));
   const int64_t E = m->K + 3;
   const int64_t fit = static_cast<int64_t>(kSlabBytes / (sizeof(double) * E * m->blocks));
-  const int64_t slab = std::max<int64_t>(1, std::min<int64_t>({C, fit, 1024}));
-  if (m->bpart_cap < slab) {
+  int64_t slab = std::max<int64_t>(1, std::min<int64_t>({C, fit, 1024}));
+  // where the device has no room for the slab, half of it, and so on
+  while (ensure_batch_partials(m, slab) != SX_OK || ensure_batch_staging(m, slab) != SX_OK) {
+    (void)hipGetLastError();  // else the next launch's check reports it
     (void)hipFree(m->d_bpart);
     m->d_bpart = nullptr;
     m->bpart_cap = 0;
-    SX_HIP(hipMalloc(&m->d_bpart, sizeof(double) * E * m->blocks * slab));
-    m->bpart_cap = slab;
+    if (slab == 1) return one_by_one(m, theta, C, propto, jacobian, lp, grad);
+    slab = (slab + 1) / 2;
   }
   return batch_call(m, theta, C, slab, true, domain_message(m->family), lp, grad,
                     [=](int n) {
@@ -1338,10 +1370,8 @@ int sx_glm_logp_grad_batch(sx_glm* m, const double* theta, int64_t C, int propto
                                                      jacobian, m->stream);
                       });
   }
-  if (C > 1) return fp64_batch(m, theta, C, propto, jacobian, lp, grad);
-  const int rc = eval(m, theta, propto, jacobian, lp, grad);
-  if (rc == SX_EDOMAIN) lp[0] = -INFINITY;
-  return rc;
+  return C > 1 ? fp64_batch(m, theta, C, propto, jacobian, lp, grad)
+               : one_by_one(m, theta, C, propto, jacobian, lp, grad);
 }
 
 int sx_glm_time_logp_grad(sx_glm* m, const double* theta, int64_t C, int iters, int warmup,

@@ -50,7 +50,9 @@ struct stream_queue {
   }
 };
 
+hipError_t g_last = hipSuccess;  // what hipGetLastError returns, once
 int g_delay_us = 0;          // before every queued operation
+int g_late_us = 3000;        // before the late words of a single evaluation
 bool g_fail_launch = false;  // kernel launches are refused
 bool g_no_store = false;     // kernels run and store nothing
 bool g_fail_pinned = false;  // no pinned memory
@@ -101,7 +103,7 @@ void put(const double* th, double* out, int D, size_t late0, size_t late1) {
   };
   for (size_t i = D + 2; i-- > 0;)
     if (i < late0 || i >= late1) one(i);
-  if (late0 < late1) pause_us(3000);
+  if (late0 < late1) pause_us(g_late_us);
   for (size_t i = late0; i < late1; ++i) one(i);
 }
 
@@ -117,10 +119,11 @@ hipError_t hipGetDevicePropertiesR0600(hipDeviceProp_tR0600* p, int) {
   p->multiProcessorCount = 256;
   return hipSuccess;
 }
+hipError_t hipGetLastError(void) { return std::exchange(g_last, hipSuccess); }
 const char* hipGetErrorString(hipError_t) { return "stand-in error"; }
 hipError_t hipMalloc(void** p, size_t n) {
   *p = nullptr;
-  if (n > g_limit - std::min(g_limit, g_used)) return hipErrorOutOfMemory;
+  if (n > g_limit - std::min(g_limit, g_used)) return g_last = hipErrorOutOfMemory;
   *p = std::calloc(1, std::max<size_t>(n, 1));
   g_dev[*p] = n;
   g_used += n;
@@ -135,7 +138,7 @@ hipError_t hipFree(void* p) {
 }
 hipError_t hipHostMalloc(void** p, size_t n, unsigned) {
   *p = nullptr;
-  if (g_fail_pinned) return hipErrorOutOfMemory;
+  if (g_fail_pinned) return g_last = hipErrorOutOfMemory;
   ++g_pinned_calls;
   *p = std::calloc(1, n);
   return hipSuccess;
@@ -196,6 +199,7 @@ static hipError_t batch(const double* theta, int64_t ts, double* out, int64_t os
                         double* scratch, int64_t per_chain, hipStream_t s, size_t late0 = 0,
                         size_t late1 = 0) {
   if (g_fail_launch) return hipErrorInvalidValue;
+  if (const hipError_t e = hipGetLastError()) return e;  // a launch's own check
   queue_of(s)->push([=] {
     for (int c = 0; c < C; ++c) {
       for (int64_t i = 0; i < per_chain; ++i) scratch[c * per_chain + i] = c;
@@ -212,6 +216,7 @@ hipError_t launch_pass_f64(int, const tile_geom&, const pass_args& a, int blocks
 hipError_t launch_eval_f64(int, const tile_geom&, const pass_args& a, const double* h_theta, int,
                            int, hipStream_t s) {
   if (g_fail_launch) return hipErrorInvalidValue;
+  if (const hipError_t e = hipGetLastError()) return e;
   const std::vector<double> th(h_theta, h_theta + a.D);  // carried by the launch
   double* out = a.out;
   queue_of(s)->push([=] { put(th.data(), out, static_cast<int>(th.size()), 2, 4); });
@@ -350,6 +355,38 @@ void failed_calls_drain() {
   sx_glm_destroy(m);
 }
 
+// Calls that need no memory of their own, or less, still run where memory is
+// refused: FP64 batches of a logistic or normal model in smaller slabs and
+// in the end chain by chain, every batch without a pinned buffer.
+void refused_memory() {
+  g_late_us = 0;
+  for (int family : {SX_LOGIT, SX_NORMAL}) {
+    // a chain's partials 4 KB (blocks = T / 4), its points and results less
+    sx_glm* m = make(family, 64 * 4 * 60, 5, 0, SX_FP64);
+    const size_t per = sizeof(double) * (m->K + 3) * m->blocks;
+    for (size_t room : {size_t(0), per, 3 * per, 20 * per, 400 * per}) {
+      g_limit = g_used + room;
+      check_batch(m, 37, 1);
+      check_batch(m, 1200, 2);
+      check_batch(m, 3, 3);
+      check_single(m, 4);
+    }
+    g_limit = SIZE_MAX;
+    check_batch(m, 1500, 5);
+    CHECK(m->bpart_cap == 1024);  // with memory, slabs of full size again
+    sx_glm_destroy(m);
+  }
+  sx_glm* models[] = {make(SX_HIER_LOGIT, 90, 3, 30, SX_FP32), make(SX_HIER_LOGIT, 90, 3, 30, SX_FP64),
+                      make(SX_LOGIT, 64, 4, 0, SX_BF16X2), make(SX_LOGIT, 64, 4, 0, SX_FP64)};
+  for (sx_glm* m : models) {
+    g_fail_pinned = true;
+    for (int64_t C : {1, 2, 40, 2000, 9000}) check_batch(m, C, 1);
+    g_fail_pinned = false;
+    for (int64_t C : {2, 2000}) check_batch(m, C, 2);
+    sx_glm_destroy(m);
+  }
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -357,6 +394,7 @@ int main(int argc, char** argv) {
   if (what == "single_fresh") single_fresh();
   else if (what == "single_slow") single_slow();
   else if (what == "failed_calls_drain") failed_calls_drain();
+  else if (what == "refused_memory") refused_memory();
   else return std::printf("unknown scenario\n"), 2;
   if (!g_bad) std::printf("ok\n");
   return g_bad != 0;

@@ -37,3 +37,10 @@ def test_failed_calls_leave_nothing_queued(check):
     """A call whose launch is refused waits for the copies it has queued: they
     read the caller's points or buffers that the next call fills."""
     check("failed_calls_drain")
+
+
+def test_batches_where_memory_is_refused(check):
+    """FP64 batches run in smaller slabs, down to chain by chain in the
+    context's own buffers, and every batch runs without a pinned buffer; the
+    refused allocation's error is not reported by a later launch."""
+    check("refused_memory")
