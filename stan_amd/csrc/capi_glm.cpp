@@ -12,6 +12,7 @@
 #include <fstream>
 #include <map>
 #include <mutex>
+#include <new>
 #include <sstream>
 #include <string>
 #include <thread>
@@ -1244,8 +1245,7 @@ int batch_call(sx_glm* m, const double* theta, int64_t C, int64_t slab, bool che
     (void)hipGetLastError();
     pinned = false;
   }
-  if (!pinned && m->bout.size() < most / sizeof(double)) m->bout.resize(most / sizeof(double));
-  const double* const out = pinned ? m->h_batch : m->bout.data();
+  std::vector<double> pageable;
   int worst = SX_OK;
   drain_on_error queued{m};
   for (int64_t b = 0; b < C; b += slab) {
@@ -1260,8 +1260,16 @@ int batch_call(sx_glm* m, const double* theta, int64_t C, int64_t slab, bool che
     SX_HIP(hipMemcpyAsync(m->d_btheta, src, n * row, hipMemcpyHostToDevice, m->stream));
     rc = enqueue(static_cast<int>(n));
     if (rc) return rc;
-    SX_HIP(hipMemcpyAsync(const_cast<double*>(out), m->d_bout, n * (row + 16),
-                          hipMemcpyDeviceToHost, m->stream));
+    if (!pinned && pageable.empty()) {  // its pages while the kernels run
+      try {
+        pageable.resize(most / sizeof(double));
+      } catch (const std::bad_alloc&) {
+        set_error("batched evaluation: out of host memory");
+        return SX_ENOMEM;
+      }
+    }
+    double* const out = pinned ? m->h_batch : pageable.data();
+    SX_HIP(hipMemcpyAsync(out, m->d_bout, n * (row + 16), hipMemcpyDeviceToHost, m->stream));
     SX_HIP(hipStreamSynchronize(m->stream));
     for (int64_t c = 0; c < n; ++c) {
       const int64_t bad = checked ? first_non_finite(th + c * D, D) : -1;

@@ -6,7 +6,6 @@
 
 #include <cstdint>
 #include <string>
-#include <vector>
 
 #include "../../include/stanx.h"
 
@@ -218,7 +217,6 @@ struct sx_glm {
   int64_t bcap = 0;
   double* h_batch = nullptr;  // pinned, of the batch calls: points, then results
   int64_t hbcap = 0;          // chains
-  std::vector<double> bout;  // pageable results of the batch calls
   double* d_bpart = nullptr;  // block partials of the FP64 batch call
   int64_t bpart_cap = 0;      // chains
   // hierarchical model

@@ -387,6 +387,26 @@ void refused_memory() {
   }
 }
 
+// Batches between the pinned buffer's limits keep no host memory: a buffer
+// held by the context costs its first call the page faults, and moves the
+// allocator's thresholds so that the caller's own result arrays of that size
+// are mapped and faulted in anew at every call.
+void nothing_kept() {
+  sx_glm* h = make(SX_HIER_LOGIT, 90, 3, 30, SX_FP32);
+  sx_glm* b = make(SX_LOGIT, 64, 40, 0, SX_BF16X2);
+  sx_glm* m = make(SX_LOGIT, 64, 40, 0, SX_FP64);
+  for (sx_glm* x : {h, b, m}) {
+    check_batch(x, 5000, 1);  // device buffers for the largest batch
+    const struct mallinfo2 a = mallinfo2();
+    check_batch(x, 300, 2);
+    check_batch(x, 350, 3);
+    const struct mallinfo2 z = mallinfo2();
+    const long kept = static_cast<long>(z.uordblks + z.hblkhd) - static_cast<long>(a.uordblks + a.hblkhd);
+    if (kept > 4096 || kept < -4096) std::printf("kept %ld bytes\n", kept), ++g_bad;
+    sx_glm_destroy(x);
+  }
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -395,6 +415,7 @@ int main(int argc, char** argv) {
   else if (what == "single_slow") single_slow();
   else if (what == "failed_calls_drain") failed_calls_drain();
   else if (what == "refused_memory") refused_memory();
+  else if (what == "nothing_kept") nothing_kept();
   else return std::printf("unknown scenario\n"), 2;
   if (!g_bad) std::printf("ok\n");
   return g_bad != 0;

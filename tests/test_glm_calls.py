@@ -44,3 +44,9 @@ def test_batches_where_memory_is_refused(check):
     context's own buffers, and every batch runs without a pinned buffer; the
     refused allocation's error is not reported by a later launch."""
     check("refused_memory")
+
+
+def test_middle_batches_keep_no_host_memory(check):
+    """Batches whose results go through pageable memory (64 KB to 1 MB) give
+    it back with the call."""
+    check("nothing_kept")
