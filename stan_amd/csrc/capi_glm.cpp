@@ -58,6 +58,11 @@ int device_cus(int* cus) {
   return SX_OK;
 }
 
+// Size of a context's pinned output buffer at least: batches whose points and
+// results each stay below it go through that buffer, so their first call pins
+// nothing (pinning took 20 of the 73 us of a context's first 8-chain batch).
+constexpr size_t kSmallBytes = size_t(64) << 10;
+
 int clamp_blocks(const sx_glm* m, int blocks) {
   const int64_t max_blocks = std::max<int64_t>(1, (m->geom.T + 3) / 4);
   return static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(blocks, max_blocks)));
@@ -547,7 +552,8 @@ int sx_glm_create_ex(sx_glm** out, int family, const double* X, const void* y, i
   if (hipMalloc(&m->d_out, sizeof(double) * (m->D + 2)) != hipSuccess) return fail(SX_ENOMEM);
   if (hipHostMalloc(&m->h_theta, sizeof(double) * (m->D + 1)) != hipSuccess) return fail(SX_ENOMEM);
   // the kernels' stores reach it while they run, whatever the process's default
-  if (hipHostMalloc(&m->h_out, sizeof(double) * (m->D + 2), hipHostMallocCoherent) != hipSuccess)
+  if (hipHostMalloc(&m->h_out, std::max(sizeof(double) * (m->D + 2), kSmallBytes),
+                    hipHostMallocCoherent) != hipSuccess)
     return fail(SX_ENOMEM);
   if (hipEventCreate(&m->ev0) != hipSuccess || hipEventCreate(&m->ev1) != hipSuccess)
     return fail(SX_EDEVICE);
@@ -1223,11 +1229,11 @@ void spread_rows(int64_t n, size_t bytes, F fn) {
 // The host copies bound a large batch (64 x 21,042 parameters, 10.8 MB each
 // way: 1670 us per call through the runtime's staging of pageable memory,
 // 1060 through a pinned buffer filled and emptied by four threads, of which
-// the kernels 88).  Small batches take the pinned buffer too (15 KB: 163 ->
-// 155 us).  Between kSmallBytes and kLargeBytes a single thread reads what a
+// the kernels 88).  Batches below kSmallBytes go through the context's pinned
+// output buffer (15 KB: 163 -> 155 us).  Between kSmallBytes and kLargeBytes a single thread reads what a
 // copy engine has just written more slowly than the runtime's staging
 // delivers it (528 KB: 302 us pageable, 307 pinned).
-constexpr size_t kSmallBytes = size_t(64) << 10, kLargeBytes = size_t(1) << 20;
+constexpr size_t kLargeBytes = size_t(1) << 20;
 
 template <class F>
 int batch_call(sx_glm* m, const double* theta, int64_t C, int64_t slab, bool checked,
@@ -1240,10 +1246,12 @@ int batch_call(sx_glm* m, const double* theta, int64_t C, int64_t slab, bool che
   const size_t most = slab * (row + 16);
   int rc = ensure_batch_staging(m, slab);
   if (rc) return rc;
-  bool pinned = most < kSmallBytes || most >= kLargeBytes;
-  if (pinned && ensure_batch_pinned(m, slab) != SX_OK) {  // refused: pageable
-    (void)hipGetLastError();
-    pinned = false;
+  double* pinned = most < kSmallBytes ? m->h_out : nullptr;
+  if (most >= kLargeBytes) {
+    if (ensure_batch_pinned(m, slab) == SX_OK)
+      pinned = m->h_batch;
+    else  // refused: pageable
+      (void)hipGetLastError();
   }
   std::vector<double> pageable;
   int worst = SX_OK;
@@ -1254,8 +1262,8 @@ int batch_call(sx_glm* m, const double* theta, int64_t C, int64_t slab, bool che
     const double* src = th;
     if (pinned) {
       spread_rows(n, n * row,
-                  [=](int64_t c) { std::memcpy(m->h_batch + c * D, th + c * D, row); });
-      src = m->h_batch;
+                  [=](int64_t c) { std::memcpy(pinned + c * D, th + c * D, row); });
+      src = pinned;
     }
     SX_HIP(hipMemcpyAsync(m->d_btheta, src, n * row, hipMemcpyHostToDevice, m->stream));
     rc = enqueue(static_cast<int>(n));
@@ -1268,7 +1276,7 @@ int batch_call(sx_glm* m, const double* theta, int64_t C, int64_t slab, bool che
         return SX_ENOMEM;
       }
     }
-    double* const out = pinned ? m->h_batch : pageable.data();
+    double* const out = pinned ? pinned : pageable.data();
     SX_HIP(hipMemcpyAsync(out, m->d_bout, n * (row + 16), hipMemcpyDeviceToHost, m->stream));
     SX_HIP(hipStreamSynchronize(m->stream));
     for (int64_t c = 0; c < n; ++c) {

@@ -202,7 +202,7 @@ struct sx_glm {
   double* d_partials = nullptr;
   double* d_out = nullptr;
   double* h_theta = nullptr;  // pinned
-  double* h_out = nullptr;    // pinned
+  double* h_out = nullptr;    // pinned: a single evaluation's or a small batch's results
   int blocks = 0, threads = 256, max_blocks = 0;
   // BF16 hi+lo layouts for batched MFMA evaluation (precision SX_BF16X2)
   int64_t Np = 0, Kp = 0;
@@ -215,7 +215,7 @@ struct sx_glm {
   double* d_btheta = nullptr;  // batched theta / out staging for the C-ABI batch call
   double* d_bout = nullptr;
   int64_t bcap = 0;
-  double* h_batch = nullptr;  // pinned, of the batch calls: points, then results
+  double* h_batch = nullptr;  // pinned, of the large batches: points, then results
   int64_t hbcap = 0;          // chains
   double* d_bpart = nullptr;  // block partials of the FP64 batch call
   int64_t bpart_cap = 0;      // chains

@@ -50,3 +50,9 @@ def test_middle_batches_keep_no_host_memory(check):
     """Batches whose results go through pageable memory (64 KB to 1 MB) give
     it back with the call."""
     check("nothing_kept")
+
+
+def test_small_batches_pin_no_memory(check):
+    """Batches below 64 KB go through pinned memory that the context has from
+    its creation."""
+    check("small_batches_pin_nothing")
