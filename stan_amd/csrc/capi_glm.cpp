@@ -1279,22 +1279,26 @@ int batch_call(sx_glm* m, const double* theta, int64_t C, int64_t slab, bool che
     double* const out = pinned ? pinned : pageable.data();
     SX_HIP(hipMemcpyAsync(out, m->d_bout, n * (row + 16), hipMemcpyDeviceToHost, m->stream));
     SX_HIP(hipStreamSynchronize(m->stream));
-    for (int64_t c = 0; c < n; ++c) {
+    // status word of a chain: 0, 1 (domain error), or 2 + the index of its
+    // first non-finite parameter; without a domain error the log density is
+    // finite
+    spread_rows(n, grad ? n * row : 0, [=](int64_t c) {
+      double* o = out + c * (D + 2);
       const int64_t bad = checked ? first_non_finite(th + c * D, D) : -1;
-      const double* o = out + c * (D + 2);
-      lp[b + c] = o[0];
-      if (bad >= 0 || o[D + 1] != 0.0) {
-        lp[b + c] = -INFINITY;
+      if (bad >= 0) o[D + 1] = 2.0 + static_cast<double>(bad);
+      lp[b + c] = o[D + 1] == 0.0 ? o[0] : -INFINITY;
+      if (grad && bad < 0) std::memcpy(grad + (b + c) * D, o + 1, row);
+    });
+    for (int64_t c = n - 1; c >= 0; --c)
+      if (lp[b + c] == -INFINITY) {  // the last one's message
+        const double status = out[c * (D + 2) + D + 1];
         worst = SX_EDOMAIN;
-        set_error(bad >= 0 ? "log_prob: parameter " + std::to_string(bad) + " is not finite"
-                           : std::string(message));
+        set_error(status < 2.0 ? std::string(message)
+                               : "log_prob: parameter " +
+                                     std::to_string(static_cast<int64_t>(status - 2.0)) +
+                                     " is not finite");
+        break;
       }
-    }
-    if (grad)
-      spread_rows(n, n * row, [=](int64_t c) {
-        if (!checked || first_non_finite(th + c * D, D) < 0)
-          std::memcpy(grad + (b + c) * D, out + c * (D + 2) + 1, row);
-      });
   }
   queued.done = true;
   return worst;

@@ -425,6 +425,39 @@ void small_batches_pin_nothing() {
   }
 }
 
+// Batches report the last chain with a domain error, give every such chain
+// -inf, and leave the gradient of a chain at a non-finite point alone (a
+// mixed-precision or hierarchical batch evaluates it).
+void batch_errors() {
+  struct {
+    sx_glm* m;
+    bool checked;
+  } models[] = {{make(SX_HIER_LOGIT, 90, 3, 30, SX_FP32), false},
+                {make(SX_LOGIT, 64, 40, 0, SX_BF16X2), false},
+                {make(SX_NORMAL, 64, 40, 0, SX_FP64), true}};
+  for (auto& x : models) {
+    const int D = static_cast<int>(x.m->D);
+    for (int64_t C : {2, 300, 9000}) {
+      std::vector<double> th = points(C, D, 1), lp(C, 7.0), g(C * D, 7.0);
+      th[0] = 1e200;  // an overflow
+      if (x.checked) th[(C - 1) * D + 3] = NAN;
+      CHECK(sx_glm_logp_grad_batch(x.m, th.data(), C, 1, 1, lp.data(), g.data()) == SX_EDOMAIN);
+      const std::string said = sx_last_error();
+      CHECK((said.find("parameter 3 is not finite") != std::string::npos) == x.checked);
+      CHECK(lp[0] == -INFINITY && g[1] == slope(th.data(), 1));
+      if (x.checked)
+        for (int i = 0; i < D; ++i) CHECK(g[(C - 1) * D + i] == 7.0);
+      CHECK((lp[C - 1] == -INFINITY) == x.checked);
+      for (int64_t c = 1; c + 1 < C; ++c) check_chain(&th[c * D], D, lp[c], &g[c * D]);
+      std::vector<double> lp2(C);
+      CHECK(sx_glm_logp_grad_batch(x.m, th.data(), C, 1, 1, lp2.data(), nullptr) == SX_EDOMAIN);
+      CHECK(lp == lp2);
+      check_batch(x.m, C, 2);
+    }
+    sx_glm_destroy(x.m);
+  }
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -435,6 +468,7 @@ int main(int argc, char** argv) {
   else if (what == "refused_memory") refused_memory();
   else if (what == "nothing_kept") nothing_kept();
   else if (what == "small_batches_pin_nothing") small_batches_pin_nothing();
+  else if (what == "batch_errors") batch_errors();
   else return std::printf("unknown scenario\n"), 2;
   if (!g_bad) std::printf("ok\n");
   return g_bad != 0;

@@ -56,3 +56,10 @@ def test_small_batches_pin_no_memory(check):
     """Batches below 64 KB go through pinned memory that the context has from
     its creation."""
     check("small_batches_pin_nothing")
+
+
+def test_batches_report_domain_errors(check):
+    """-inf for every chain with a domain error, the last one's message, the
+    gradient of a chain at a non-finite point left alone; on one thread and on
+    several."""
+    check("batch_errors")
