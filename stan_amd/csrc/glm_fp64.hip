@@ -309,7 +309,7 @@ template <int FAM, bool ARG>
 hipError_t launch_pass(const tile_geom& g, const pass_args& a, const theta_of<ARG>& ta,
                        int blocks, int threads, hipStream_t s) {
   if constexpr (!ARG)
-    if (chains_pass_fits(g, a, threads)) return launch_pass_f64_chains(FAM, g, a, blocks, s);
+    if (chains_pass_fits(FAM, g, a, threads)) return launch_pass_f64_chains(FAM, g, a, blocks, s);
   return g.prefetch ? launch_fam<FAM, 1, ARG>(g.smax, a, ta, blocks, threads, s)
                     : launch_fam<FAM, 0, ARG>(g.smax, a, ta, blocks, threads, s);
 }

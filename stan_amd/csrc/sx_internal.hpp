@@ -66,17 +66,30 @@ hipError_t launch_pass_f64(int family, const tile_geom& g, const pass_args& a,
 // the same partials, bit for bit, as the single-chain pass.
 hipError_t launch_pass_f64_chains(int family, const tile_geom& g, const pass_args& a, int blocks,
                                   hipStream_t s);
-// Whether a batch takes it.  It needs L <= 4 lanes per row (a DPP row of 16
-// lanes then holds rows of one column group), a wave's worth of chains for
-// each of its four waves, and work to outweigh its longer latency.  Measured
-// us, single-chain pass over a grid of chains -> this one: N = 1e6, K = 100,
-// 32 chains 2678 -> 848, 8 chains 741 -> 365; N = 200,003, K = 60, 32 chains
-// 281 -> 137; around the line N = 20,000, K = 20, 32 chains 24.9 -> 23.7, N =
-// 50,000, K = 20, 8 chains 18.7 -> 18.3; below it N = 10,000, K = 50, 8
-// chains 13.0 -> 19.5, N = 3000, K = 37, 32 chains 11.1 -> 17.0.
-inline bool chains_pass_fits(const tile_geom& g, const pass_args& a, int threads) {
-  return a.chains >= 8 && threads == 256 && g.L <= 4 && g.S > 0 &&
-         a.N * a.K * a.chains >= (int64_t(1) << 23);
+// Whether a batch takes it instead of the single-chain pass over a grid of
+// chains.  It needs L <= 4 lanes per row (a DPP row of 16 lanes then holds
+// rows of one column group): never above K = 128, whose layouts have 8 lanes
+// or more, and not where the tuner, which times single evaluations, chose 8.
+//  - Its groups of eight chains must be filled, more than five on average: a
+//    group with one chain costs nearly as much as a full one.  us per call,
+//    grid / this: 9 chains, logistic N = 900,000, K = 1, 10 chains 77 / 88, at
+//    2^26 products K = 2 1.29 times, K = 10 1.07 times the grid's; 12 chains
+//    0.76 .. 1.02 times, 16 chains 0.69 .. 0.83.  From 2^26 products the
+//    reads saved carry a nearly empty group too where rows are wide or the
+//    link is cheap: 9 chains, K >= 32 0.91 .. 1.0, normal K <= 10 0.75 .. 0.89.
+//  - N K chains from 2^23 (L = 1), 1.5 2^23 (L = 2) or 3 2^23 (L = 4): its
+//    latency grows with the lanes of a row.  8, 16 and 64 chains, times the
+//    grid's, at 2^23, 2^24, 2^25: K = 20 0.97 0.88 0.83; K = 64 1.08 0.97
+//    0.82; K = 127 1.12 1.05 0.93.
+// Far above the lines: N = 1e6, K = 100, 32 chains 2678 / 848, 8 chains
+// 741 / 365; N = 200,003, K = 60, 32 chains 281 / 137.
+inline bool chains_pass_fits(int family, const tile_geom& g, const pass_args& a, int threads) {
+  if (a.chains < 8 || threads != 256 || g.L > 4 || g.S <= 0) return false;
+  const int64_t products = a.N * a.K * a.chains;
+  const int groups = (a.chains + 7) / 8;
+  const bool filled = a.chains > 5 * groups;
+  const bool reads = products >= (int64_t(1) << 26) && (family == SX_NORMAL || a.K >= 32);
+  return products >= (int64_t(g.L == 1 ? 2 : g.L == 2 ? 3 : 6) << 22) && (filled || reads);
 }
 
 // One evaluation at a host theta: pass and reduction, with theta carried by

@@ -458,6 +458,49 @@ void batch_errors() {
   }
 }
 
+// Which batches take the several-chains FP64 pass: on either side of each
+// line where it was measured against the single-chain pass.
+void chains_rule() {
+  struct {
+    int family;
+    int64_t N;
+    int K, L, C;
+    bool fits;
+  } cases[] = {
+      {SX_LOGIT, 200003, 60, 2, 32, true},   {SX_LOGIT, 1000000, 100, 4, 8, true},
+      {SX_LOGIT, 10000000, 100, 4, 7, false}, {SX_LOGIT, 1000000, 100, 8, 32, false},
+      {SX_NORMAL, 1000000, 200, 8, 32, false},
+      // groups of eight with few chains
+      {SX_LOGIT, 900000, 1, 1, 10, false},   {SX_LOGIT, 900000, 1, 1, 16, true},
+      {SX_LOGIT, 3728270, 2, 1, 9, false},   {SX_LOGIT, 745654, 10, 1, 10, false},
+      {SX_LOGIT, 300000, 10, 1, 11, true},   {SX_LOGIT, 300000, 10, 1, 17, true},
+      {SX_LOGIT, 240000, 32, 1, 9, true},    {SX_LOGIT, 200000, 32, 1, 9, false},
+      {SX_NORMAL, 900000, 10, 1, 9, true},   {SX_NORMAL, 700000, 10, 1, 9, false},
+      // work
+      {SX_LOGIT, 53000, 20, 1, 8, true},     {SX_LOGIT, 52000, 20, 1, 8, false},
+      {SX_LOGIT, 25000, 64, 2, 8, true},     {SX_LOGIT, 24000, 64, 2, 8, false},
+      {SX_LOGIT, 25000, 127, 4, 8, true},    {SX_LOGIT, 24000, 127, 4, 8, false},
+      // the forms the GPU tests compare bit for bit with single evaluations
+      {SX_LOGIT, 120011, 9, 1, 8, true},     {SX_LOGIT, 70001, 13, 1, 11, true},
+      {SX_LOGIT, 61007, 37, 2, 17, true},    {SX_LOGIT, 60005, 60, 4, 8, true},
+      {SX_LOGIT, 33333, 63, 4, 13, true},    {SX_LOGIT, 21000, 128, 4, 16, true},
+      {SX_LOGIT, 66000, 29, 4, 33, true},    {SX_LOGIT, 20001, 32, 1, 18, true},
+      {SX_LOGIT, 100033, 17, 2, 8, true},    {SX_LOGIT, 400001, 3, 2, 12, true},
+      {SX_LOGIT, 32003, 101, 4, 8, true},    {SX_LOGIT, 236001, 32, 1, 9, true},
+      {SX_NORMAL, 1700003, 4, 1, 10, true},
+  };
+  for (const auto& c : cases) {
+    sx::tile_geom g = sx::make_geom(c.N, c.K, c.L, 32);
+    sx::pass_args a{};
+    a.N = c.N;
+    a.K = c.K;
+    a.chains = c.C;
+    if (sx::chains_pass_fits(c.family, g, a, 256) != c.fits || sx::chains_pass_fits(c.family, g, a, 64))
+      std::printf("family %d N %ld K %d L %d chains %d\n", c.family, static_cast<long>(c.N), c.K, c.L, c.C),
+          ++g_bad;
+  }
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -469,6 +512,7 @@ int main(int argc, char** argv) {
   else if (what == "nothing_kept") nothing_kept();
   else if (what == "small_batches_pin_nothing") small_batches_pin_nothing();
   else if (what == "batch_errors") batch_errors();
+  else if (what == "chains_rule") chains_rule();
   else return std::printf("unknown scenario\n"), 2;
   if (!g_bad) std::printf("ok\n");
   return g_bad != 0;

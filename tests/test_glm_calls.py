@@ -63,3 +63,8 @@ def test_batches_report_domain_errors(check):
     gradient of a chain at a non-finite point left alone; on one thread and on
     several."""
     check("batch_errors")
+
+
+def test_which_batches_share_tiles(check):
+    """The several-chains FP64 pass is taken where it is the faster one."""
+    check("chains_rule")
