@@ -153,7 +153,8 @@ __global__ __launch_bounds__(256) void glm_pass_f64(pass_args a, theta_of<ARG> t
     double rr = 0.0, term = 0.0;
     if (valid) {
       if (FAM == SX_LOGIT) {
-        stanx::math::sx_logit_row(e, yv != 0.0 ? 1.0 : -1.0, &term, &rr);
+        // with four slots the link is most of the work, and registers are free
+        stanx::math::sx_logit_row<(SMAX > 4)>(e, yv != 0.0 ? 1.0 : -1.0, &term, &rr);
       } else {
         const double d = yv - e;
         rr = d;
