@@ -182,17 +182,33 @@ int create_batch(sx_nuts_batch** out, sx_glm* m, const sx_nuts_config* cfg, int6
     //  - above 8192 coordinates always (a vector pass costs about as much
     //    as the gradient).  Hierarchical D = 21,042, 64 chains, ms in all:
     //    1008 unbounded, 954 with 6, 908 with 4, 950 with 3;
-    //  - below, for gradients under about 50 us (N K chains <= 2^30,
-    //    FP32 / BF16) and enough work per step for one chain to stand out
-    //    (D >= 32, D chains >= 2048).  ms unbounded / with 4: logistic
-    //    20000 x 100, 256 chains 164 / 149; x 200 239 / 208; 64 chains
-    //    127 / 119; hierarchical FP32, 64 chains, D = 612 74 / 63,
-    //    D = 1812 105 / 82, D = 7722 149 / 122.
+    //  - below, for FP32 / BF16 gradients, with enough work per step for
+    //    one chain to stand out (D >= 32, D chains >= 2048), enough chains
+    //    for one of them to be closing a subtree at most steps
+    //    (hierarchical 8 from D = 500 on and 16 below, the others 24), and a
+    //    gradient that is cheap for the chains it serves: N K chains <=
+    //    2^30, and per chain at most 2^17 rows (hierarchical 2^21) once the
+    //    chains are padded to the tile the kernels work on.  ms unbounded /
+    //    with 4: logistic 20000 x 100, 256 chains 164 / 149; x 200 239 /
+    //    208; 64 chains 127 / 119; D = 512, 24 chains 412 / 409; D = 256, 24
+    //    chains 137 / 133; 100000 x 64, 128 chains 47.7 / 46.3;
+    //    hierarchical, 64 chains, D = 612 74 / 63, D = 1812 105 / 82, D =
+    //    7722 149 / 122; 16 chains, D = 260 220 / 209; 8 chains, D = 510
+    //    254 / 253, D = 1012 276 / 264, D = 6342 668 / 642.
     // On the other side of those lines: 1e6 x 100, 24 chains 271 / 286;
     // hierarchical 2^30.6 123 / 127; D = 11, 16 chains 21.3 / 24.2;
     // D = 104, 16 chains 41.6 / 42.7; FP64 40000 x 50, 32 chains
-    // 132 / 135.  STANX_NUTS_PHASE_BUDGET=n sets it (n >= 1).
+    // 132 / 135; BF16 D = 512, 4 chains 354 / 371, D = 256, 16 chains 208 /
+    // 211; hierarchical 1 chain, D = 2142 209 / 219, D = 6342 419 / 437, 4
+    // chains 565 / 568, D = 260, 8 chains 191.1 / 191.6; 200000 x 100, 32
+    // chains 39.1 / 40.9; hierarchical, 840,000 rows, D = 6342, 8 chains
+    // 162 / 171.  STANX_NUTS_PHASE_BUDGET=n sets it (n >= 1).
+    const bool hier = m->family == SX_HIER_LOGIT;
+    const int64_t enough = !hier ? 24 : D >= 500 ? 8 : 16;
+    const int64_t padded =
+        hier ? (chains + 31) / 32 * 32 : sx::mx_chain_pad(m, static_cast<int>(chains));
     const bool cheap = grad_precision != SX_FP64 && D >= 32 && D * chains >= 2048 &&
+                       chains >= enough && m->N * padded <= chains << (hier ? 21 : 17) &&
                        static_cast<double>(m->N) * m->K * chains <= 1073741824.0;
     b->a.phase_budget = D > 8192 || cheap ? 4 : 4096;
     if (const char* e = std::getenv("STANX_NUTS_PHASE_BUDGET"))

@@ -191,6 +191,7 @@ struct sx_glm;
 namespace sx {
 int mx_enqueue(sx_glm* m, mx_workspace& w, const double* d_theta, int C, double* d_out,
                int propto, int jacobian, hipStream_t stream);
+int mx_chain_pad(const sx_glm* m, int C);
 int hier_prepare(sx_glm* m, hier_workspace& w, int C);
 int mx_autotune(sx_glm* m);
 int plain_enqueue(sx_glm* m, const double* d_theta, double* d_out, double* partials, int propto,
