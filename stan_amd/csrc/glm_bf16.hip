@@ -855,8 +855,12 @@ __global__ __launch_bounds__(64 * NW) void glm_mfma32_adj(mx_args a) {
 // slices are combined in slice order: a fixed order that depends on N, K and
 // the split count only.  RB = 4 up to 64 chains, where one block per chain
 // leaves most CUs idle (64 chains, 192 splits, K = 468: 11.2 us with RB = 1,
-// 9.1 with 4); more chains fill the chip, and whole rows read better (256
-// chains, 512 splits, K = 100: 16.6 us with RB = 1, 19.4 with 4).
+// 9.1 with 4; whole evaluations of 24 and 64 chains, 200,000 x 256, 68.1 and
+// 74.4 -> 64.8 and 72.3); more chains fill the chip, and whole rows read
+// better (256 chains, 512 splits, K = 100: 16.6 us with RB = 1, 19.4 with 4).
+// A row of 32 columns is one cache line, which four blocks would each fetch:
+// RB = 4 up to 16 chains there (100,000 x 30, 8, 24 and 64 chains 24.2, 24.2
+// and 25.2 us with RB = 1, 24.0, 24.8 and 26.7 with 4).
 template <int FAM, int RB>
 __global__ __launch_bounds__(1024 / RB) void mx_reduce(mx_args a, pass_args pa) {
   __shared__ double red[4096 / RB];  // [slice][column of the block]
@@ -1049,7 +1053,7 @@ hipError_t launch_mfma_pass(int family, const double* theta, int64_t D, int C, c
     default: return hipErrorInvalidValue;
   }
   if (e != hipSuccess) return e;
-  const bool few = C <= 64;
+  const bool few = C <= (a.Kp > 32 ? 64 : 16);
   if (family == SX_LOGIT && few)
     hipLaunchKernelGGL((mx_reduce<SX_LOGIT, 4>), dim3(C * 4), dim3(256), 0, s, a, pa);
   else if (family == SX_LOGIT)
