@@ -114,7 +114,7 @@ int64_t footprint_of(const sx_job_spec& s) {
     if (prec == SX_FP32 && K <= 31)  // the split copy of X (3 BF16 terms)
       bytes += 48 * (N + 32) * sx::hier_x6_chunks(static_cast<int>(K));
     const int64_t chunks = ceil_div(N, sx::kHierChunkMin) + s.J;  // any autotuned chunk size
-    bytes += chunks * 16 + (s.J + 1) * 8;
+    bytes += chunks * static_cast<int64_t>(sizeof(sx::hier_chunk)) + (s.J + 1) * 8;
     bytes += 8 * ((K + 3) * std::max<int64_t>(1, chunks) + (2 * K + 5) * s.J) * (C + 1);
     if (prec == SX_FP32 && K <= 31) bytes += 192 * s.J * (C + 1);  // split coefficients
   } else {
