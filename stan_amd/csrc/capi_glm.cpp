@@ -994,6 +994,26 @@ int mx_enqueue(sx_glm* m, mx_workspace& w, const double* d_theta, int C, double*
   return SX_OK;
 }
 
+// Row splits to time, as target tiles per split: 4 to 128 tiles, and those
+// that give half, one and two splits per CU, so that the workgroups of one or
+// two chain blocks fill whole rounds of the device (N = 2e5, K = 256: 200
+// splits make 400 workgroups for 256 chains, 1.6 rounds of 256 CUs; 256
+// splits make two).  Each split count once.
+static std::vector<int> mx_split_targets(const sx_glm* m, int cus) {
+  const int64_t n_tiles = m->Np / 32, per = std::max(1, cus);
+  std::vector<int> targets, seen;
+  for (int64_t t : {int64_t(4), int64_t(8), int64_t(16), int64_t(32), int64_t(64), int64_t(128),
+                    (2 * n_tiles + per - 1) / per, (n_tiles + per - 1) / per,
+                    (n_tiles + 2 * per - 1) / (2 * per)}) {
+    t = std::max<int64_t>(1, t);
+    const int sp = mx_splits(m, t);
+    if (std::find(seen.begin(), seen.end(), sp) != seen.end()) continue;
+    seen.push_back(sp);
+    targets.push_back(static_cast<int>(t));
+  }
+  return targets;
+}
+
 // Launch shape of the batched MFMA pass, timed on the device at context
 // creation: the kernel variant (one wave per 32-chain block; a pair of
 // waves split by k where Kp / 32 is even and at most 8; or, for Kp <= 128,
@@ -1038,24 +1058,9 @@ int mx_autotune(sx_glm* m) {
   const int kq = static_cast<int>(m->Kp / 32);
   int best_v = 0, best_t = 8;
   double best_ms = 1e30;
-  // Targets: 4 to 128 tiles per split, and those that give half, one and two
-  // splits per CU, so that the workgroups of one or two chain blocks fill
-  // whole rounds of the device (N = 2e5, K = 256: 200 splits make 400
-  // workgroups for 256 chains, 1.6 rounds of 256 CUs; 256 splits make two).
-  // Each split count is timed once.
   int cus = 0;
   if (rc == SX_OK) rc = device_cus(&cus);
-  const int64_t n_tiles = m->Np / 32;
-  std::vector<int> targets, seen;
-  for (int64_t t : {int64_t(4), int64_t(8), int64_t(16), int64_t(32), int64_t(64), int64_t(128),
-                    (2 * n_tiles + cus - 1) / std::max(1, cus), (n_tiles + cus - 1) / std::max(1, cus),
-                    (n_tiles + 2 * cus - 1) / std::max(1, 2 * cus)}) {
-    t = std::max<int64_t>(1, t);
-    const int sp = mx_splits(m, t);
-    if (std::find(seen.begin(), seen.end(), sp) != seen.end()) continue;
-    seen.push_back(sp);
-    targets.push_back(static_cast<int>(t));
-  }
+  const std::vector<int> targets = mx_split_targets(m, cus);
   for (int v = 0; v <= 2 && rc == SX_OK; ++v) {
     if (v == 1 && (m->Kp > 256 || kq % 2 != 0)) continue;
     if (v == 2 && kq > 4) continue;

@@ -501,6 +501,32 @@ void chains_rule() {
   }
 }
 
+// The row splits that are timed: every tile in one of them, each count once,
+// and half, one and two per CU among them where the rows suffice.
+void split_targets() {
+  for (int64_t tiles : {1, 7, 8, 63, 255, 256, 257, 1506, 6250, 6251, 31250, 99999})
+    for (int cus : {0, 64, 228, 256, 304}) {
+      sx_glm m;
+      m.Np = 32 * tiles;
+      std::vector<int> splits;
+      for (int t : sx::mx_split_targets(&m, cus)) {
+        const int s = sx::mx_splits(&m, t);
+        CHECK(t >= 1 && s >= 8 && s <= 512 && s % 8 == 0);
+        CHECK((tiles + s - 1) / s * s >= tiles);
+        for (int o : splits) CHECK(o != s);
+        splits.push_back(s);
+      }
+      // a whole number of tiles per split rounds the count down, by less
+      // than one tile's worth, and a multiple of 8 up
+      for (int want : {cus / 2, cus, 2 * cus})
+        if (want >= 8 && want <= 512 && tiles >= 100 * want) {
+          bool near = false;
+          for (int s : splits) near |= s > want - want / 50 - 1 && s <= want + 7;
+          CHECK(near);
+        }
+    }
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -513,6 +539,7 @@ int main(int argc, char** argv) {
   else if (what == "small_batches_pin_nothing") small_batches_pin_nothing();
   else if (what == "batch_errors") batch_errors();
   else if (what == "chains_rule") chains_rule();
+  else if (what == "split_targets") split_targets();
   else return std::printf("unknown scenario\n"), 2;
   if (!g_bad) std::printf("ok\n");
   return g_bad != 0;

@@ -68,3 +68,7 @@ def test_batches_report_domain_errors(check):
 def test_which_batches_share_tiles(check):
     """The several-chains FP64 pass is taken where it is the faster one."""
     check("chains_rule")
+
+
+def test_row_splits_that_are_timed(check):
+    check("split_targets")

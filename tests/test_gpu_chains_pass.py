@@ -40,3 +40,30 @@ def test_either_pass_is_the_single_evaluation(family, N, K, L, cap, blocks, C):
     assert abs(lp[0] - lp_r) <= TOL * max(1.0, abs(lp_r))
     assert np.linalg.norm(g[0] - g_r) <= TOL * max(1.0, np.linalg.norm(g_r))
     m.close()
+
+
+@pytest.mark.parametrize("family,N,K,L,cap", [(S.LOGIT, 60_000, 20, 1, 20), (S.NORMAL, 40_000, 60, 4, 16),
+                                              (S.LOGIT, 50_001, 33, 2, 20)])
+def test_device_chains_share_tiles(family, N, K, L, cap, monkeypatch):
+    """16 device chains, whose captured steps hold the several-chains pass, are
+    bitwise those of batches of 2 (the single-chain pass), and of the same 16
+    with the steps launched directly."""
+    print(f"device chains family={family} N={N} K={K} L={L}", flush=True)
+    assert 2 * N * K < 1 << 23 and 16 * N * K >= {1: 2, 2: 3, 4: 6}[L] << 22
+    d = W.logistic(N, K, 1.0 / np.sqrt(K), 0.5, seed=K) if family == S.LOGIT \
+        else W.normal(N, K, seed=K)
+    m = S.GlmModel(family, d["X"], d["y"], prior=d["prior"],
+                   tuning=dict(lanes_per_row=L, slots_cap=cap, blocks=512, autotune=0))
+    cfg = dict(random_seed=5, num_warmup=15, num_samples=10, max_depth=5, save_warmup=1)
+    keys = ("draws", "rows", "status", "stepsize", "inv_metric", "n_grad")
+    many = S.hmc_nuts_diag_e_adapt_batch(m, 16, chain=1, **cfg)
+    assert np.all(many["status"] == 0)
+    for first in (1, 9, 15):
+        two = S.hmc_nuts_diag_e_adapt_batch(m, 2, chain=first, **cfg)
+        for key in keys:
+            np.testing.assert_array_equal(two[key], many[key][first - 1:first + 1])
+    monkeypatch.setenv("STANX_BATCH_NO_GRAPH", "1")
+    direct = S.hmc_nuts_diag_e_adapt_batch(m, 16, chain=1, **cfg)
+    for key in keys:
+        np.testing.assert_array_equal(direct[key], many[key])
+    m.close()
