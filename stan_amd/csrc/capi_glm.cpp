@@ -723,16 +723,18 @@ int take_words(sx_glm* m, const double* w, size_t n, double* dst,
                std::chrono::steady_clock::time_point start) {
   bool synced = false;
   unsigned spins = 0;
-  const auto unset = [w](size_t i) {
-    return __atomic_load_n(reinterpret_cast<const uint64_t*>(w + i), __ATOMIC_ACQUIRE) == kUnset;
-  };
   for (size_t i = 0; i < n;) {
-    const size_t e = std::min(n, i + 64);
+    constexpr size_t kBlock = 64;
+    uint64_t v[kBlock];  // what is copied is what was seen to be stored
+    const size_t count = std::min(n - i, kBlock);
     bool any = false;
-    for (size_t k = i; k < e; ++k) any |= unset(k);
+    for (size_t k = 0; k < count; ++k) {
+      v[k] = __atomic_load_n(reinterpret_cast<const uint64_t*>(w + i + k), __ATOMIC_ACQUIRE);
+      any |= v[k] == kUnset;
+    }
     if (!any) {
-      if (dst) std::memcpy(dst + i, w + i, (e - i) * sizeof(double));
-      i = e;
+      if (dst) std::memcpy(dst + i, v, count * sizeof(double));
+      i += count;
     } else if (synced) {
       set_error("log_prob: the device stored no result");
       return SX_EDEVICE;
@@ -814,10 +816,11 @@ int eval(sx_glm* m, const double* theta, int propto, int jacobian, double* lp,
   if (rc == SX_OK)
     rc = take_words(m, m->h_out + 1, head - 1, grad, start);
   if (rc == SX_OK) rc = take_words(m, m->h_out, 1, lp, start);
-  if (rc == SX_OK) rc = take_words(m, m->h_out + D + 1, 1, nullptr, start);
+  double status = 0.0;
+  if (rc == SX_OK) rc = take_words(m, m->h_out + D + 1, 1, &status, start);
   if (rc) return rc;
   queued.done = true;
-  if (m->h_out[D + 1] != 0.0) {
+  if (status != 0.0) {
     set_error(domain_message(m->family));
     return SX_EDOMAIN;
   }
