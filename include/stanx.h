@@ -395,7 +395,11 @@ int sx_nuts_batch_create(sx_nuts_batch** out, sx_glm* m,
                          int grad_precision, const double* inits,
                          const double* inv_metric);
 /* Advance all chains by up to max_steps lockstep gradient steps (stops
- * early once every chain has finished).                                 */
+ * early once every chain has finished).  max_steps bounds the work of one
+ * call; it is no measure of progress: a chain that has much to do between
+ * two gradients may pass over some steps (environment variable
+ * STANX_NUTS_PHASE_BUDGET=n: after n phases), so how many draws a number of
+ * steps gives depends on the schedule; the draws themselves do not.     */
 /* Steps run as replays of a captured HIP graph of 16 steps; with the
  * environment variable STANX_BATCH_NO_GRAPH=1 at create they are launched
  * directly instead (same kernels and results; for kernel tracers).     */

@@ -613,7 +613,7 @@ int sx_glm_create_ex(sx_glm** out, int family, const double* X, const void* y, i
   if (rc == SX_OK && precision == SX_BF16X2) {
     m->Np = (N + 31) / 32 * 32;
     // a multiple of 32 up to 256; above, of 64 (the adjoint's column
-    // blocks of 256 + 64 j)
+    // blocks of 128, a last one of 64)
     m->Kp = K <= 256 ? std::max<int64_t>(32, (K + 31) / 32 * 32) : (K + 63) / 64 * 64;
     const size_t elems = static_cast<size_t>(m->Np) * m->Kp;
     if (hipMalloc(&m->d_Xh, elems * 2) != hipSuccess || hipMalloc(&m->d_Xl, elems * 2) != hipSuccess ||

@@ -10,11 +10,12 @@
 // each wave loads a 64-row-block tile of X into registers (one 512-byte
 // coalesced load per slot), forms eta with an L-lane reduction,
 // evaluates the link, and accumulates x * r into per-lane FP64 registers.
-// Block partials are summed in a fixed order by a second one-block launch,
-// so results are bitwise reproducible, and that launch adds the priors and
-// the log-Jacobian and writes lp and the gradient.  This replaces the two GEMV passes over X that the reference's
-// CPU GLM performs per gradient (Stan Math bernoulli_logit_glm_lpmf /
-// normal_id_glm_lpdf, reached through src/stan/model/gradient.hpp:21-35).
+// Block partials are summed in a fixed order by a second launch of a few
+// blocks per chain, so results are bitwise reproducible, and that launch adds
+// the priors and the log-Jacobian and writes lp and the gradient.  This
+// replaces the two GEMV passes over X that the reference's CPU GLM performs
+// per gradient (Stan Math bernoulli_logit_glm_lpmf / normal_id_glm_lpdf,
+// reached through src/stan/model/gradient.hpp:21-35).
 #include <hip/hip_runtime.h>
 
 #include <cmath>

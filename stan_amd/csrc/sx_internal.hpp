@@ -25,7 +25,7 @@ void set_error(const std::string& msg);
 // Geometry of the lane-slot tiled X layout used by the bulk passes.
 // A wave-tile holds R = 64 / L rows; each row is split across L lanes and
 // each lane holds S = ceil(K / L) columns ("slots").  Element (row, col)
-// of the tile t lives at  t*S*64 + (col / L)*64 + (row % R)*L + col % L,
+// of the tile t lives at  t*S*64 + (col / L)*64 + (col % L)*R + row % R,
 // so slot j of all 64 lanes is one contiguous 512-byte (FP64) segment.
 struct tile_geom {
   int L = 1;       // lanes per row (power of two, <= 64)
